@@ -55,6 +55,18 @@ static unsigned resident_grid(F* kernel, int block, int requested) {
         (void)hipGetLastError();
         nb = 1;
     }
+    // The LDS is handed out in units of 1280 bytes (160 KB / 128), which the
+    // occupancy query does not round up to: a P2G of 14,720 bytes got 11
+    // workgroups per CU where 10 fit, so one in eleven waited for a whole
+    // round (340 us instead of 277 for 2.1M particles).
+    hipFuncAttributes fa;
+    if (hipFuncGetAttributes(&fa, (const void*)kernel) == hipSuccess) {
+        const size_t unit = 1280, per_cu = 160 * 1024;
+        const size_t bytes = (fa.sharedSizeBytes + unit - 1) / unit * unit;
+        if (bytes > 0 && per_cu / bytes >= 1) nb = nb < (int)(per_cu / bytes) ? nb : (int)(per_cu / bytes);
+    } else {
+        (void)hipGetLastError();
+    }
     const int grid = nb * device_cus();
     cache[key] = grid;
     return (unsigned)grid;
@@ -96,13 +108,26 @@ struct G2PWaves {
 // Syz(b,c)), so they run 5 waves per SIMD (measured: the two-kernel slab
 // step 1.412 -> 1.398 ms and the 256-scene APIC batch 2.354 -> 2.313 ms
 // from 4 waves; 3 -> 4 waves had taken APIC P2G from 0.674 to 0.616 ms).
-// The 7-value P2G and the cubic stencil keep the compiler's allocation.
+// The 7-value P2G of the narrower stencils keeps the compiler's allocation;
+// the cubic one (matrix cores) runs what its LDS leaves room for, which also
+// keeps its accumulators out of the AGPRs.
 #ifndef MPM_P2G_WAVES
 #define MPM_P2G_WAVES 5
 #endif
+// The P2G whose cell sums run on the matrix cores: the cubic stencil's.
+// Measured, scan against products: cubic APIC, 8 particles per cell (two
+// balls, 141k) 56.9 -> 31.8 us; quadratic APIC at 4-8 per cell (256-scene batch)
+// 733 against 733 us, PIC-FLIP at 2 per cell (2.1M slab) 251 against 277 us:
+// the scan of a quadratic stencil has 27 nodes instead of 64, its products
+// fill 108 of 256 results, and few particles share a cell's flush.
+template <int INTERP, int MODE>
+struct P2GMatrix {
+    static constexpr bool value = INTERP == MPM_INTERP_CUBIC_BSPLINE && MODE != 1;
+};
 template <int INTERP, int MODE>
 struct P2GWaves {
-    static constexpr int value = (MODE == 0 || INTERP == MPM_INTERP_CUBIC_BSPLINE) ? 1 : MPM_P2G_WAVES;
+    static constexpr bool cubic = INTERP == MPM_INTERP_CUBIC_BSPLINE;
+    static constexpr int value = cubic ? (MODE == 2 ? 3 : (MODE == 1 ? 1 : 2)) : (MODE == 0 ? 1 : MPM_P2G_WAVES);
 };
 
 // ------------------------------------------------------------------ keys
@@ -641,6 +666,245 @@ __device__ __forceinline__ void seg_scan(float (&v)[N], const SegPlan& sp) {
     if (sp.s31) MPM_SCAN_STEP(NV, v, "row_bcast:31 row_mask:0xc", sp.f31);
 }
 
+// Cell sums on the matrix cores.  With the per-axis factors of one particle,
+// a component k of its contribution to node (a, b, c) of its stencil is
+//   RX_k(a) Ny(b) Nz(c) + Nx(a) [RY_k(b) Nz(c) + Ny(b) RZ_k(c)]
+// (momentum m w (v + C (x_i - x_p)) and force vs grad w split by axis: RX_k =
+// m Nx (v_k + C_k0 dx) + vs_k0 dNx, RY_k = m Ny C_k1 dy + vs_k1 dNy, RZ_k
+// likewise; the mass, k = 0, has RX_0 = m Nx and nothing else).  Over rows
+// (a, k) and columns (b, c) that is a product of rank 4, one
+// v_mfma_f32_16x16x4f32 per particle:
+//   A[(a, k)][0] = RX_k(a)   B[0][(b, c)] = Ny(b) Nz(c)
+//   A[(a, k)][r] = Nx(a) if k = r, else 0
+//                            B[r][(b, c)] = RY_r(b) Nz(c) + Ny(b) RZ_r(c)
+// and the particles of one cell, which are consecutive, add up in the
+// accumulator, in FP32 as before.  A cubic stencil fills the 16x16 result, a
+// quadratic one 12x9 of it, a linear one 8x4.
+// Each lane writes its own particle's factors into an LDS record (kRec
+// particles at a time; an odd number of words apart: no bank conflicts), and
+// every lane reads, for each particle of the batch, the two words its A and B
+// elements are.  The result lane (a, (b, c)) holds the node's four values, so
+// a cell is added into the LDS tile with one 16-byte read and write per lane.
+//
+// The segmented DPP scan that this replaces spent 4 or 7 values x up to 6
+// scan steps on each of the stencil's nodes and a read-add-write per node.
+template <int W, bool MOM>
+struct CellRec {
+    static constexpr int RX = 0, NX = 4 * W, ZERO = 5 * W, BX = 5 * W + 1, PX = BX + 4 * W * W;
+    static constexpr int WORDS = PX + (MOM ? 3 * W : 0);
+    static constexpr int STRIDE = WORDS | 1;
+};
+#ifndef MPM_REC
+#define MPM_REC 32
+#endif
+constexpr int kRec = MPM_REC;  // particles per record batch
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+// A wave's LDS instructions execute in order; this keeps the compiler from
+// moving them across (lanes read words that other lanes wrote before it).
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
+// The lane's record words (A, B, the second A of MOM) and its place in the
+// result: tile node (from the cell's first) and whether it holds one.
+template <int W, bool MOM, int T>
+struct CellLane {
+    int a, b, p, node;
+    bool out;
+    __device__ __forceinline__ explicit CellLane(int lane) {
+        using R = CellRec<W, MOM>;
+        const int i = lane & 15, r = lane >> 4, row = i >> 2, k = i & 3;
+        const int j = i < W * W ? i : 0;
+        a = row >= W ? R::ZERO : (r == 0 ? R::RX + i : (k == r ? R::NX + row : R::ZERO));
+        b = R::BX + r * W * W + j;
+        p = row < W && r == 0 && k > 0 ? R::PX + 3 * row + k - 1 : R::ZERO;
+        out = r < W && i < W * W;
+        node = out ? (j % W * T + j / W) * T + r : 0;
+    }
+};
+
+// One lane's record: factors of the components (mass or 0, then three) per
+// axis node; px: the momentum factors of MOM.
+template <int W, bool MOM>
+__device__ __forceinline__ void cell_record(float* q, const float (&mx)[W], const float (&rx)[3][W],
+                                            const float (&ry)[3][W], const float (&rz)[3][W], const float (&Nx)[W],
+                                            const float (&Ny)[W], const float (&Nz)[W], const float (&px)[3][W]) {
+    using R = CellRec<W, MOM>;
+    q[R::ZERO] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        q[R::RX + 4 * j] = mx[j];
+        q[R::NX + j] = Nx[j];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            q[R::RX + 4 * j + 1 + k] = rx[k][j];
+            if (MOM) q[R::PX + 3 * j + k] = px[k][j];
+        }
+#pragma unroll
+        for (int c = 0; c < W; ++c) {
+            q[R::BX + j * W + c] = Ny[j] * Nz[c];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                q[R::BX + ((k + 1) * W + j) * W + c] = fmaf(ry[k][j], Nz[c], Ny[j] * rz[k][c]);
+        }
+    }
+}
+
+// A wave's lanes of one item (the first cnt are active) added into the tile:
+// records and products, kRec particles at a time.  tails: the last lane of
+// each cell; cell: the lane's cell's first tile node.  MOM adds a second
+// accumulator, (0, momentum) = the words PX times Ny Nz, into tile2.
+template <int W, bool MOM, int T>
+__device__ __forceinline__ void cell_scatter(float* rec, const CellLane<W, MOM, T>& L, int lane, int cnt,
+                                             uint64_t tails, int cell, const float (&mx)[W], const float (&rx)[3][W],
+                                             const float (&ry)[3][W], const float (&rz)[3][W], const float (&Nx)[W],
+                                             const float (&Ny)[W], const float (&Nz)[W], const float (&px)[3][W],
+                                             f4* tile, f4* tile2) {
+    constexpr int ST = CellRec<W, MOM>::STRIDE;
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, acc2 = acc;
+    for (int l0 = 0; l0 < cnt; l0 += kRec) {
+        wave_lds_order();
+        if (lane >= l0 && lane < l0 + kRec && lane < cnt)
+            cell_record<W, MOM>(rec + (lane - l0) * ST, mx, rx, ry, rz, Nx, Ny, Nz, px);
+        wave_lds_order();
+        const int n = cnt - l0 < kRec ? cnt - l0 : kRec;
+        const float *qa = rec + L.a, *qb = rec + L.b, *qp = rec + L.p;
+        for (int p0 = 0; p0 < n; p0 += 4) {
+            float a[4], b[4], pa[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {  // records past n hold old words: read, not used
+                a[u] = qa[u * ST];
+                b[u] = qb[u * ST];
+                if (MOM) pa[u] = qp[u * ST];
+            }
+            qa += 4 * ST;
+            qb += 4 * ST;
+            if (MOM) qp += 4 * ST;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int p = p0 + u;
+                if (p >= n) break;
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u], acc, 0, 0, 0);
+                if (MOM) acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[u], b[u], acc2, 0, 0, 0);
+                if ((tails >> (l0 + p)) & 1ull) {
+                    const int off = __builtin_amdgcn_readlane(cell, l0 + p);
+                    if (L.out) {
+                        f4* const q = tile + off + L.node;
+                        *q = *q + acc;
+                        if (MOM) {
+                            f4* const q2 = tile2 + off + L.node;
+                            *q2 = *q2 + acc2;
+                        }
+                    }
+                    acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+                    if (MOM) acc2 = acc;
+                }
+            }
+        }
+    }
+    wave_lds_order();
+}
+
+// The factors (above) of one particle's folded-grid contributions
+// (particlesToGrid, src/apic_mpm_solver3d.cu:245-304, with p + dt f summed
+// per node): mass m w and m w (v + C (x_i - x_p)) + vs grad w, vs = dt tau.
+template <int W>
+__device__ __forceinline__ void folded_factors(float m, const float (&vel)[3], const float (&Cm)[3][3],
+                                               const float (&vs)[3][3], const float (&dxn)[3][W],
+                                               const float (&Nx)[W], const float (&Ny)[W], const float (&Nz)[W],
+                                               const float (&dNx)[W], const float (&dNy)[W], const float (&dNz)[W],
+                                               float (&mNx)[W], float (&rx)[3][W], float (&ry)[3][W],
+                                               float (&rz)[3][W]) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        mNx[j] = m * Nx[j];
+        const float mNy = m * Ny[j], mNz = m * Nz[j];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            rx[k][j] = fmaf(mNx[j], vel[k] + Cm[k][0] * dxn[0][j], vs[k][0] * dNx[j]);
+            ry[k][j] = fmaf(mNy, Cm[k][1] * dxn[1][j], vs[k][1] * dNy[j]);
+            rz[k][j] = fmaf(mNz, Cm[k][2] * dxn[2][j], vs[k][2] * dNz[j]);
+        }
+    }
+}
+
+template <int W>
+__device__ __forceinline__ float pick(const float (&v)[W], int i) {
+    float r = v[0];
+#pragma unroll
+    for (int j = 1; j < W; ++j) r = i == j ? v[j] : r;
+    return r;
+}
+__device__ __forceinline__ float lane_value(float v, int src) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src));
+}
+// Clears the factors of a lane that scatter_one takes (on = false).
+template <int W>
+__device__ __forceinline__ void keep_finite(bool on, float (&mx)[W], float (&rx)[3][W], float (&ry)[3][W],
+                                            float (&rz)[3][W], float (&px)[3][W]) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        mx[j] = on ? mx[j] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            rx[k][j] = on ? rx[k][j] : 0.0f;
+            ry[k][j] = on ? ry[k][j] : 0.0f;
+            rz[k][j] = on ? rz[k][j] : 0.0f;
+            px[k][j] = on ? px[k][j] : 0.0f;
+        }
+    }
+}
+
+// One particle (lane src of the wave) added into the tile node by node, one
+// lane per node.  The products above multiply zeros into the components that
+// a term does not belong to, so a particle with a non-finite stress or affine
+// velocity would spread it to the others (0 * inf): it comes here instead,
+// where each component sees its own terms only.
+template <int INTERP, int APIC, int T>
+__device__ __forceinline__ void scatter_one(const SceneDev& S, f4* tile, f4* tile2, bool apart, int ox, int oy, int oz,
+                                            int lane, int src, const float (&xp)[3], float mp, const float (&vp)[3],
+                                            const float (&Cp)[3][3], const float (&vsp)[3][3]) {
+    constexpr int W = Stencil<INTERP>::W;
+    float x[3], v[3], C[3][3], t[3][3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        x[k] = lane_value(xp[k], src);
+        v[k] = lane_value(vp[k], src);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            C[k][j] = APIC ? lane_value(Cp[k][j], src) : 0.0f;
+            t[k][j] = lane_value(vsp[k][j], src);
+        }
+    }
+    const float m = lane_value(mp, src);
+    if (lane >= W * W * W) return;
+    const int a = lane / (W * W), b = (lane / W) % W, c = lane % W;
+    int bx, by, bz;
+    float Nx[W], Ny[W], Nz[W], dNx[W], dNy[W], dNz[W];
+    axis_weights<INTERP>(x[0], S.ox, S.h, S.inv_h, bx, Nx, dNx);
+    axis_weights<INTERP>(x[1], S.oy, S.h, S.inv_h, by, Ny, dNy);
+    axis_weights<INTERP>(x[2], S.oz, S.h, S.inv_h, bz, Nz, dNz);
+    const int gi = bx + a, gj = by + b, gk = bz + c;
+    const float nx = pick<W>(Nx, a), ny = pick<W>(Ny, b), nz = pick<W>(Nz, c);
+    const float gw[3] = {pick<W>(dNx, a) * ny * nz, nx * pick<W>(dNy, b) * nz, nx * ny * pick<W>(dNz, c)};
+    const float dx[3] = {(S.ox + S.h * (float)gi) - x[0], (S.oy + S.h * (float)gj) - x[1],
+                         (S.oz + S.h * (float)gk) - x[2]};
+    const float mw = m * ((nx * ny) * nz);
+    f4* const q = tile + (((gk - oz) * T + (gj - oy)) * T + (gi - ox));
+    f4* const q2 = tile2 + (((gk - oz) * T + (gj - oy)) * T + (gi - ox));
+    f4 val = *q, val2 = apart ? *q2 : val;
+    val[0] += mw;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float p = mw * (APIC ? v[k] + ((C[k][0] * dx[0] + C[k][1] * dx[1]) + C[k][2] * dx[2]) : v[k]);
+        const float f = (t[k][0] * gw[0] + t[k][1] * gw[1]) + t[k][2] * gw[2];
+        val[1 + k] += apart ? f : p + f;
+        val2[1 + k] += apart ? p : 0.0f;
+    }
+    *q = val;
+    if (apart) *q2 = val2;
+}
+
 template <int INTERP, int APIC, int MODE, bool BATCH>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWaves<INTERP, MODE>::value))) k_p2g(SceneDev S0, ParticlesDev P0, ItemsDev I,
                                             const SceneEntry* __restrict__ tab) {
@@ -649,9 +913,18 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWave
     constexpr int TN = T * T * T;
     constexpr int NF = MODE == 0 ? 7 : (MODE == 1 ? 1 : 4);
     static_assert(MODE != 2 || APIC, "the folded grid serves APIC only");
-    __shared__ float tile[NF * TN];
+    // the cell sums on the matrix cores: the tile's nodes hold mass and
+    // momentum plus force (MODE 2) or force (MODE 0), with the momentum in a
+    // second tile; else one plane per value and the segmented scan
+    constexpr bool MM = P2GMatrix<INTERP, MODE>::value;
+    constexpr bool MOM = MODE == 0 && !APIC;
+    __shared__ float tile[MM ? 1 : NF * TN];
+    __shared__ f4 mtile[MM ? TN : 1];
+    __shared__ f4 mtile2[MM && MODE == 0 ? TN : 1];
+    __shared__ float rec[MM ? kRec * CellRec<W, MOM>::STRIDE : 1];
     const uint32_t nitems = *I.count;
     const int lane = threadIdx.x;
+    const CellLane<W, MOM, T> L(lane);
     for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
         // a fused batch step: scenes whose last step already scattered this P2G
         if (BATCH && tab[I.scene[it]].prescat != 0u) continue;
@@ -669,7 +942,14 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWave
                 }
             continue;
         }
-        for (int q = lane; q < NF * TN; q += 64) tile[q] = 0.0f;
+        if constexpr (MM) {
+            for (int q = lane; q < TN; q += 64) {
+                mtile[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (MODE == 0) mtile2[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        } else {
+            for (int q = lane; q < NF * TN; q += 64) tile[q] = 0.0f;
+        }
         __syncthreads();
         for (uint32_t base = g.s; base < g.e; base += 64) {
             const uint32_t i = base + lane;
@@ -678,7 +958,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWave
             // segment structure of this chunk (inactive lanes form their own tail segment)
             const uint32_t key = active ? I.sorted_keys[ic] : 0xFFFFFFFFu;
             const uint32_t prev = __shfl_up(key, 1, 64);
-            const SegPlan sp = seg_plan(__ballot(lane == 0 || prev != key), active, lane);
+            const uint64_t heads = __ballot(lane == 0 || prev != key);
+            const SegPlan sp = seg_plan(heads, active, lane);
             const bool writer = sp.writer;
             const uint32_t praw = I.perm[ic];
             const uint32_t p = praw - pbase;
@@ -695,7 +976,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWave
             const int lx = bx - g.ox, ly = by - g.oy, lz = bz - g.oz;
             // tile cell of the stencil's first node; node (a, b, c) is at
             // tq[(c * T + b) * T + a] (constant offsets)
-            float* const tq = tile + ((lz * T + ly) * T + lx);
+            float* const tq = tile + (MM ? 0 : (lz * T + ly) * T + lx);
             const float m = active ? P.m[p] : 0.0f;
             if (MODE == 1) {
 #pragma unroll
@@ -744,6 +1025,47 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWave
                     dxn[1][j] = (S.oy + S.h * (float)(by + j)) - x1;
                     dxn[2][j] = (S.oz + S.h * (float)(bz + j)) - x2;
                 }
+            }
+            if constexpr (MM) {
+                const int cnt = (int)(g.e - base < 64u ? g.e - base : 64u);
+                const uint64_t tails = (heads >> 1) | (1ull << (cnt - 1));
+                const int cell = (lz * T + ly) * T + lx;
+                // finite? (a sum of some of the terms is not exactly if one is not)
+                float fin = (vs[0][1] + vs[0][2]) + (vs[1][1] + vs[1][2]) + vs[2][2];
+                if (APIC) fin += (Cm[0][1] + Cm[0][2]) + (Cm[1][1] + Cm[1][2]) + (Cm[2][1] + Cm[2][2]);
+                const uint64_t odd = __ballot(active && !__builtin_isfinite(fin));
+                const bool on = !((odd >> lane) & 1ull);
+                const float xp[3] = {x0, x1, x2}, vk[3] = {v0, v1, v2};
+                for (uint64_t left = odd; left; left &= left - 1)
+                    scatter_one<INTERP, APIC, T>(S, mtile, mtile2, MODE == 0, g.ox, g.oy, g.oz, lane,
+                                                 __builtin_ctzll(left), xp, m, vk, Cm, vs);
+                const float mo = on ? m : 0.0f;
+                float mNx[W], rx[3][W], ry[3][W], rz[3][W], px[3][W];
+                if constexpr (MODE == 2) {
+                    folded_factors<W>(mo, vk, Cm, vs, dxn, Nx, Ny, Nz, dNx, dNy, dNz, mNx, rx, ry, rz);
+                } else {
+                    if constexpr (APIC) {  // momentum and force apart: one set of sums each
+                        const float none[3][3] = {}, zero[W] = {};
+                        folded_factors<W>(mo, vk, Cm, none, dxn, Nx, Ny, Nz, dNx, dNy, dNz, mNx, rx, ry, rz);
+                        if (odd) keep_finite<W>(on, mNx, rx, ry, rz, px);
+                        cell_scatter<W, MOM, T>(rec, L, lane, cnt, tails, cell, zero, rx, ry, rz, Nx, Ny, Nz, px,
+                                                mtile2, mtile2);
+                    }
+#pragma unroll
+                    for (int j = 0; j < W; ++j) {
+                        mNx[j] = mo * Nx[j];
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            px[k][j] = mNx[j] * vk[k];
+                            rx[k][j] = vs[k][0] * dNx[j];
+                            ry[k][j] = vs[k][1] * dNy[j];
+                            rz[k][j] = vs[k][2] * dNz[j];
+                        }
+                    }
+                }
+                if (odd) keep_finite<W>(on, mNx, rx, ry, rz, px);
+                cell_scatter<W, MOM, T>(rec, L, lane, cnt, tails, cell, mNx, rx, ry, rz, Nx, Ny, Nz, px, mtile, mtile2);
+                continue;
             }
             if constexpr (MODE == 2) {
                 // the folded grid: momentum plus force of node (a, b, c) as
@@ -848,7 +1170,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWave
             bool any = false;
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
-                const float val = tile[f * TN + q];
+                float val;
+                if constexpr (MM) val = MODE == 2 || f == 0 ? mtile[q][f] : (f < 4 ? mtile2[q][f] : mtile[q][f - 3]);
+                else val = tile[f * TN + q];
                 if (val != 0.0f) {
                     unsafeAtomicAdd(&S.grid[(int64_t)f * S.plane + ni], val);
                     any = true;
@@ -1498,16 +1822,6 @@ __device__ __forceinline__ void folded_cell_sums(float* tq, const SegPlan& sp, f
 // T^3 nodes from (ox, oy, oz); null for no tile) is added into that LDS
 // tile, which the item flushes with the rest; a particle that stayed in its
 // key block has its whole stencil there.  Other nodes take global atomics.
-template <int W>
-__device__ __forceinline__ float pick(const float (&v)[W], int i) {
-    float r = v[0];
-#pragma unroll
-    for (int j = 1; j < W; ++j) r = i == j ? v[j] : r;
-    return r;
-}
-__device__ __forceinline__ float lane_value(float v, int src) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src));
-}
 template <int INTERP, int T>
 __device__ __forceinline__ void scatter_moved(const SceneDev& S, float* grid, uint32_t* touched, float* ot, int ox,
                                               int oy, int oz, uint64_t moved, int lane, const float (&xn)[3], float m,
