@@ -345,7 +345,8 @@ MPM_API int mpm_get_stats(void* handle, mpm_stats* out);
 
 /* ------------------------------------------------------------- profiling */
 /* enable: 0 off; 1 every kernel group (two events around each launch group:
- * about 30 per step, which add ~0.1 ms of stream gaps per step); 2 only the
+ * about 30 per step, which add ~0.1 ms of stream gaps per step; a scene below
+ * 2^20 particles then sorts in full every step); 2 only the
  * item kernels p2g and g2p, or the fused g2p2g (2-4 events per step), and
  * the store reorder. */
 MPM_API int mpm_profile_enable(void* handle, int enable);

@@ -374,6 +374,7 @@ int relayout(Batch& b) {
         b.I.plan = b.plan;
         b.I.moves = b.moves_dev;
         b.I.move_cap = b.move_cap;
+        b.I.move_mask = kMoveLists - 1;
     }
     b.snap_ok = false;  // slots and keys laid out anew
     if (!b.tune_fixed) {

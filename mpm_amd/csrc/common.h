@@ -117,6 +117,8 @@ struct SceneEntry {
 // step (its G2P took 1.31 ms instead of 0.96).
 constexpr int kMoveMin = 16384;   // capacity of all sub-lists: max(kMoveMin, particles / 8)
 constexpr int kMoveLists = 64;
+constexpr int kSmallLists = 16;   // of a scene below kIncMinParticles, each of small_list_cap(n) entries
+__host__ __device__ inline uint32_t small_list_cap(int64_t n) { return (uint32_t)((n + kSmallLists - 1) / kSmallLists); }
 constexpr int kMoveCountStride = 64;  // words between two sub-list counters
 constexpr int kIncTile = 2048;    // snapshot entries per merge workgroup
 constexpr int kIncStage = 512;    // removals or insertions a merge workgroup ranks in LDS
@@ -125,6 +127,7 @@ enum PlanWord {
     kPlanIncSteps = 2,  // steps sorted by the update since creation
     kPlanCap = 3,       // capacity of one sub-list
     kPlanOverflow = 4,  // a sub-list overflowed, or a snapshot tile drew more than kIncStage entries
+    kPlanMoves = 5,     // entries of the move list of the last sort
     kPlanLists = 64,    // the sub-list counters: word kPlanLists + r * kMoveCountStride
     kPlanWords = kPlanLists + kMoveLists * kMoveCountStride
 };
@@ -167,4 +170,8 @@ struct ItemsDev {
     uint32_t* plan;
     const MoveList* moves;  // device copy of the list's pointers
     uint32_t move_cap;
+    // sub-lists in use - 1; a small scene's kSmallLists are followed by one
+    // that takes what a full one cannot (spill), for every particle
+    uint32_t move_mask;
+    uint32_t spill;
 };

@@ -215,6 +215,242 @@ __global__ void __launch_bounds__(kIncWG) k_inc_merge(const uint32_t* __restrict
     }
 }
 
+// ------------------------------------------------------------ small scenes
+// The same update in one launch.  A small scene's step is a chain of short
+// launches, so here every workgroup reads the whole move list (a few percent
+// of the particles) and keeps what falls into its tile, instead of passes
+// that bucket the list first: the removals and insertions before the tile
+// give its offset, a scan over the tile's positions the place of every entry
+// in it.  Insertions at one place are put into scratch in arbitrary order,
+// then ranked among themselves.  The list holds every particle, so there is
+// no overflow and no full sort to launch beside it.
+// What bounds it: the list's entries times the tiles (12 bytes each, from
+// L2); the host takes the radix sort instead where that is the larger (see
+// run_sort_small).  Measured at 16,384 particles: six radix launches of 41 us
+// and their gaps and a grid clear of 5 us before, one of 8.6 us for both now.
+constexpr int kMatch = 512;  // of a tile's insertions, those kept in LDS
+
+// Number of tile entries below (key, slot).
+__device__ __forceinline__ uint32_t place_in_tile(const uint32_t* sk, const uint32_t* sp, uint32_t cnt, uint32_t k,
+                                                  uint32_t s) {
+    uint32_t lo = 0, hi = cnt;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (entry_less(sk[mid], sp[mid], k, s)) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Clear of the touched blocks of a grid, 8 consecutive blocks per wave.
+__device__ __forceinline__ void clear_blocks(const GridClear& C, int64_t wave) {
+    const int lane = threadIdx.x & 63;
+    const int64_t b0 = wave * 8;
+    uint64_t todo = __ballot(lane < 8 && b0 + lane < C.nsb && C.touched[b0 + lane] != 0u);
+    unsigned long long cnt = 0;
+    while (todo) {
+        const int64_t b = b0 + __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const int64_t ni = b * 64 + lane;
+        cnt += (unsigned long long)__popcll(__ballot(C.grid[ni] > 0.0f));
+        for (int f = 0; f < C.nfields; ++f) C.grid[(int64_t)f * C.plane + ni] = 0.0f;
+        if (lane == 0) C.touched[b] = 0u;
+    }
+    if (C.active && cnt && lane == 0) atomicAdd(C.active, cnt);
+}
+
+__global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restrict__ plan, MoveList L,
+                                                        const uint32_t* __restrict__ snap_k,
+                                                        const uint32_t* __restrict__ snap_p, uint32_t n,
+                                                        uint32_t tiles, uint32_t* __restrict__ out_k,
+                                                        uint32_t* __restrict__ out_p, uint32_t* tmp_k,
+                                                        uint32_t* tmp_p, GridClear C) {
+    if (blockIdx.x >= tiles) {
+        clear_blocks(C, (int64_t)(blockIdx.x - tiles) * (kIncWG / 64) + (threadIdx.x >> 6));
+        return;
+    }
+    constexpr int TILE = kUpdateTile, IPT = TILE / kIncWG;
+    __shared__ uint32_t sk[TILE], sp[TILE];
+    __shared__ uint32_t ins[TILE + 1];        // insertions at each place of the tile (TILE: after its last entry)
+    __shared__ uint32_t before[TILE + 1];     // removals (low 11 bits) and insertions before each place
+    __shared__ uint32_t gone[TILE / 32];      // removed positions
+    __shared__ uint32_t mk[kMatch], ms[kMatch], place[kMatch];  // the tile's insertions and their places
+    __shared__ uint32_t nmatch, ws[kIncWG / 64];
+    static_assert(TILE <= 1024, "removals of a tile take 11 bits of `before`");
+    const uint32_t t = blockIdx.x, tid = threadIdx.x;
+    const uint32_t i0 = t * TILE, cnt = n - i0 < TILE ? n - i0 : TILE;
+    const bool last = t + 1 == tiles;
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const uint32_t i = tid + r * kIncWG;
+        if (i < cnt) {
+            sk[i] = snap_k[i0 + i];
+            sp[i] = snap_p[i0 + i];
+        }
+        ins[i] = 0u;
+    }
+    if (tid < TILE / 32) gone[tid] = 0u;
+    if (tid == 0) {
+        ins[TILE] = 0u;
+        nmatch = 0u;
+    }
+    const uint32_t nk = last ? 0u : snap_k[i0 + TILE], np = last ? 0u : snap_p[i0 + TILE];
+    __syncthreads();
+    const uint32_t fk = sk[0], fp = sp[0];
+    // whether (k, s) goes into this tile: -1 an earlier one, 0 this, 1 a later one
+    auto side = [&](uint32_t k, uint32_t s) -> int {
+        if (t > 0 && entry_less(k, s, fk, fp)) return -1;
+        return !last && !entry_less(k, s, nk, np) ? 1 : 0;
+    };
+    // every list entry, once over the workgroup: a wave takes four sub-lists
+    // side by side (their loads in flight together), then all take what did
+    // not fit into them
+    const uint32_t cap = small_list_cap(n);
+    constexpr uint32_t WAVES = kIncWG / 64, OWN = kSmallLists / WAVES;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63u;
+    const uint32_t spilled = plan[kPlanLists + kSmallLists * kMoveCountStride];
+    uint32_t own[OWN], longest = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < OWN; ++u) {
+        const uint32_t c = plan[kPlanLists + (wave + u * WAVES) * kMoveCountStride];
+        own[u] = c < cap ? c : cap;
+        longest = own[u] > longest ? own[u] : longest;
+    }
+    auto for_list = [&](auto&& fn) {
+        for (uint32_t q = lane; q < longest; q += 64u) {
+            uint32_t k[OWN], s[OWN], pos[OWN];
+#pragma unroll
+            for (uint32_t u = 0; u < OWN; ++u) {
+                const uint32_t j = (wave + u * WAVES) * cap + q;
+                if (q < own[u]) {
+                    k[u] = L.key[j];
+                    s[u] = L.slot[j];
+                    pos[u] = L.pos[j];
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < OWN; ++u)
+                if (q < own[u]) fn(k[u], s[u], pos[u]);
+        }
+        for (uint32_t q = tid; q < spilled; q += kIncWG) {
+            const uint32_t j = kSmallLists * cap + q;
+            fn(L.key[j], L.slot[j], L.pos[j]);
+        }
+    };
+    uint32_t db = 0, ib = 0;
+    for_list([&](uint32_t k, uint32_t s, uint32_t pos) {
+        if (pos < i0) ++db;
+        else if (pos - i0 < cnt) atomicOr(&gone[(pos - i0) >> 5], 1u << ((pos - i0) & 31u));
+        const int w = side(k, s);
+        if (w < 0) ++ib;
+        if (w == 0) {
+            const uint32_t q = atomicAdd(&nmatch, 1u);
+            if (q < kMatch) {
+                mk[q] = k;
+                ms[q] = s;
+            } else {
+                atomicAdd(&ins[place_in_tile(sk, sp, cnt, k, s)], 1u);
+            }
+        }
+    });
+    __syncthreads();
+    const uint32_t nm = nmatch;
+    for (uint32_t q = tid; q < (nm < kMatch ? nm : kMatch); q += kIncWG) {
+        place[q] = place_in_tile(sk, sp, cnt, mk[q], ms[q]);
+        atomicAdd(&ins[place[q]], 1u);
+    }
+    __syncthreads();
+    uint32_t dtot, itot, dsum, isum;
+    block_exclusive_scan(db, ws, dtot);
+    block_exclusive_scan(ib, ws, itot);
+    // thread tid scans places IPT * tid ..
+    uint32_t d[IPT], c[IPT];
+    uint32_t ds = 0, is = 0;
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const uint32_t i = tid * IPT + r;
+        d[r] = ds;
+        c[r] = is;
+        ds += (gone[i >> 5] >> (i & 31u)) & 1u;
+        is += ins[i];
+    }
+    const uint32_t dpre = block_exclusive_scan(ds, ws, dsum);
+    const uint32_t ipre = block_exclusive_scan(is, ws, isum);
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) before[tid * IPT + r] = (dpre + d[r]) | ((ipre + c[r]) << 11);
+    if (tid == 0) before[TILE] = dsum | (isum << 11);
+    __syncthreads();
+    const uint32_t base = i0 - dtot + itot;
+    // first place in the new order of what is inserted at place l
+    auto bucket = [&](uint32_t l) -> uint32_t { return base + l - (before[l] & 2047u) + (before[l] >> 11); };
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const uint32_t i = tid + r * kIncWG;
+        if (i >= cnt || ((gone[i >> 5] >> (i & 31u)) & 1u)) continue;
+        const uint32_t dst = bucket(i) + ins[i];
+        if (dst < n) {  // always, for a list that matches the snapshot
+            out_k[dst] = sk[i];
+            out_p[dst] = sp[i];
+        }
+    }
+    if (nm == 0u) return;  // uniform
+    __syncthreads();       // sk is free: from here on the bucket cursors
+    uint32_t* const cur = sk;
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) cur[tid + r * kIncWG] = 0u;
+    // the places were found with sk; entries beyond kMatch need it again, so
+    // their place is found in the snapshot in memory
+    __shared__ uint32_t cur_last;
+    if (tid == 0) cur_last = 0u;
+    __syncthreads();
+    auto for_matches = [&](auto&& fn) {
+        if (nm <= kMatch) {
+            for (uint32_t q = tid; q < nm; q += kIncWG) fn(mk[q], ms[q], place[q]);
+        } else {
+            for_list([&](uint32_t k, uint32_t s, uint32_t) {
+                if (side(k, s) == 0) fn(k, s, place_in_tile(snap_k + i0, snap_p + i0, cnt, k, s));
+            });
+        }
+    };
+    for_matches([&](uint32_t k, uint32_t s, uint32_t l) {
+        const uint32_t u = atomicAdd(l < TILE ? &cur[l] : &cur_last, 1u);
+        const uint32_t dst = bucket(l) + u;
+        if (dst >= n) return;
+        uint32_t* const ok = ins[l] == 1u ? out_k : tmp_k;
+        uint32_t* const op = ins[l] == 1u ? out_p : tmp_p;
+        ok[dst] = k;
+        op[dst] = s;
+    });
+    __syncthreads();
+    for_matches([&](uint32_t k, uint32_t s, uint32_t l) {
+        const uint32_t c0 = ins[l], b0 = bucket(l);
+        if (c0 == 1u || b0 + c0 > n) return;
+        uint32_t rank = 0;
+        for (uint32_t u = 0; u < c0; ++u) rank += entry_less(tmp_k[b0 + u], tmp_p[b0 + u], k, s) ? 1u : 0u;
+        out_k[b0 + rank] = k;
+        out_p[b0 + rank] = s;
+    });
+}
+
+__global__ void k_update_init(uint32_t* plan, MoveList* dev, MoveList L) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < (uint32_t)kPlanWords) plan[i] = 0u;
+    if (i == 0u) *dev = L;
+}
+void launch_update_init(uint32_t* plan, MoveList* dev, const MoveList& L, hipStream_t st) {
+    hipLaunchKernelGGL(k_update_init, dim3((kPlanWords + 255) / 256), dim3(256), 0, st, plan, dev, L);
+}
+
+void launch_sort_update(const uint32_t* plan, const MoveList& L, const uint32_t* snap_k, const uint32_t* snap_p,
+                        int64_t n, uint32_t* out_k, uint32_t* out_p, uint32_t* tmp_k, uint32_t* tmp_p,
+                        const GridClear& clear, hipStream_t st) {
+    const uint32_t tiles = (uint32_t)((n + kUpdateTile - 1) / kUpdateTile);
+    const int64_t waves = (clear.nsb + 7) / 8;
+    const uint32_t extra = (uint32_t)((waves + kIncWG / 64 - 1) / (kIncWG / 64));
+    hipLaunchKernelGGL(k_sort_update, dim3(tiles + extra), dim3(kIncWG), 0, st, plan, L, snap_k, snap_p, (uint32_t)n,
+                       tiles, out_k, out_p, tmp_k, tmp_p, clear);
+}
+
 uint32_t inc_tiles(int64_t n) { return (uint32_t)(n / kIncTile + 1); }
 
 void launch_inc_set(uint32_t* plan, uint32_t snap_ok, hipStream_t st) {

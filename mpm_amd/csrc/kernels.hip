@@ -208,7 +208,13 @@ __global__ void __launch_bounds__(kScanWG) k_item_count(const uint32_t* __restri
                                                         uint32_t* __restrict__ plan) {
     __shared__ uint32_t ws[kScanWG / 64];
     if (plan && blockIdx.x == 0) {
-        if (threadIdx.x < kMoveLists) plan[kPlanLists + threadIdx.x * kMoveCountStride] = 0u;
+        if (threadIdx.x < kMoveLists) {  // one wave
+            uint32_t moves = plan[kPlanLists + threadIdx.x * kMoveCountStride];
+            plan[kPlanLists + threadIdx.x * kMoveCountStride] = 0u;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) moves += __shfl_xor(moves, off, 64);
+            if (threadIdx.x == 0) plan[kPlanMoves] = moves;
+        }
         if (threadIdx.x == 0) {
             plan[kPlanIncSteps] += plan_incremental(plan) ? 1u : 0u;
             plan[kPlanSnapOk] = 1u;
@@ -1221,8 +1227,9 @@ void launch_p2g(const SceneDev& S, const ParticlesDev& P, const ItemsDev& I, int
 // kMoveLists), one counter atomic per wave, then each moved lane writes
 // (new key, slot, old sorted position) at its rank.  Past the sub-list's
 // capacity nothing is stored and the overflow word sends the next step to
-// the full sort.  In two halves, so that a kernel can issue the atomic
-// early and use its result late (the wave need not wait for it).
+// the full sort; a small scene's entry goes to the list behind the others.
+// In two halves, so that a kernel can issue the atomic early and use its
+// result late (the wave need not wait for it).
 struct MoveTicket {
     uint64_t mask;  // the wave's moved lanes
     uint32_t base;  // the leader lane's atomic result
@@ -1232,7 +1239,7 @@ __device__ __forceinline__ MoveTicket move_begin(const ItemsDev& I, bool moved) 
     MoveTicket t;
     t.mask = __ballot(moved);
     t.base = 0;
-    t.list = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (uint32_t)(kMoveLists - 1);
+    t.list = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & I.move_mask;
     if (t.mask == 0ull) return t;
     const int lane = threadIdx.x & 63;
     if (lane == __ffsll((unsigned long long)t.mask) - 1)
@@ -1248,6 +1255,12 @@ __device__ __forceinline__ void move_end(const ItemsDev& I, const MoveTicket& t,
         const uint32_t idx = base + (uint32_t)__popcll(t.mask & ((1ull << lane) - 1ull));
         if (idx < I.move_cap) {
             const size_t e = (size_t)t.list * I.move_cap + idx;
+            I.moves->key[e] = key;
+            I.moves->slot[e] = slot;
+            I.moves->pos[e] = pos;
+        } else if (I.spill) {
+            const size_t e = (size_t)kSmallLists * I.move_cap +
+                             atomicAdd(&I.plan[kPlanLists + kSmallLists * kMoveCountStride], 1u);
             I.moves->key[e] = key;
             I.moves->slot[e] = slot;
             I.moves->pos[e] = pos;
@@ -2976,6 +2989,14 @@ void launch_debug_svd(const float* A, int64_t n, float* U, float* s, float* V, h
     hipLaunchKernelGGL(k_debug_svd, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, A, n, U, s, V);
 }
 
+__global__ void k_copy_u32(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, int64_t n) {
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+void launch_copy_u32(const uint32_t* src, uint32_t* dst, int64_t n, hipStream_t st) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_copy_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, src, dst, n);
+}
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, int64_t n) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;

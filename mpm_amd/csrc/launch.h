@@ -45,6 +45,23 @@ void launch_inc_prepare(uint32_t* plan, const MoveList& L, const uint32_t* snap_
                         hipStream_t st);
 void launch_inc_merge(const uint32_t* plan, const MoveList& L, const uint32_t* snap_k, const uint32_t* snap_p,
                       int64_t n, uint32_t* out_k, uint32_t* out_p, hipStream_t st);
+// The update of a scene below kIncMinParticles in one launch: its move list
+// has room for every particle, so it always applies while the snapshot is the
+// previous step's order.  tmp_k/tmp_p: n words each of
+// scratch.  clear (nsb > 0): the same launch clears that grid (touched
+// blocks, as launch_clear), which nothing in the update reads.
+struct GridClear {
+    float* grid = nullptr;
+    uint32_t* touched = nullptr;
+    int64_t plane = 0, nsb = 0;
+    int nfields = 0;
+    unsigned long long* active = nullptr;
+};
+void launch_sort_update(const uint32_t* plan, const MoveList& L, const uint32_t* snap_k, const uint32_t* snap_p,
+                        int64_t n, uint32_t* out_k, uint32_t* out_p, uint32_t* tmp_k, uint32_t* tmp_p,
+                        const GridClear& clear, hipStream_t st);
+void launch_update_init(uint32_t* plan, MoveList* dev, const MoveList& L, hipStream_t st);  // empty list, no snapshot
+constexpr int kUpdateTile = 1024;  // snapshot entries per workgroup of it
 // Sizes of the update's buffers for n particles: snapshot tiles (the tile
 // arrays hold 2 * (tiles + 1) words each) and the capacity of one sub-list
 // (the list arrays hold kMoveLists times that).
@@ -162,6 +179,7 @@ void launch_batch_health(const SceneEntry* tab, const uint32_t* key_offsets, int
 void launch_count_escaped(const uint32_t* sorted_keys, int64_t n, uint32_t escape_key, unsigned long long* out,
                           hipStream_t st);
 void launch_debug_svd(const float* A, int64_t n, float* U, float* s, float* V, hipStream_t st);
+void launch_copy_u32(const uint32_t* src, uint32_t* dst, int64_t n, hipStream_t st);
 void launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t st);
 
 }  // namespace mpm

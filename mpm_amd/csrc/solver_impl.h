@@ -131,6 +131,12 @@ struct Solver {
     MoveList moves{};
     MoveList* moves_dev = nullptr;  // device copy of `moves` (the kernels' view)
     uint32_t move_cap = 0;          // capacity of one sub-list (also in the plan words)
+    // a scene below kIncMinParticles: the update in one launch
+    // (launch_sort_update) on the same snapshot, plan words and list (its own
+    // sub-lists; allocated at the first fused step); moves_seen: the list's
+    // length in a recent step, or -1
+    bool small_sort = false;
+    int64_t moves_seen = -1;
     // how often the update ran lately: the incremental-sort count read back
     // every few steps through pinned memory (never waited for); mostly
     // updates -> the full sort's launches use fewer passes (few_passes)
@@ -155,6 +161,7 @@ struct Solver {
     decltype(SceneDev::grid) grid2 = nullptr;
     decltype(SceneDev::touched) touched2 = nullptr;
     decltype(SceneDev::grid) graph_grid = nullptr;  // the grid buffer the captured step uses
+    bool graph_small = false;  // the captured step's sort is the small update
     // member of a batch that fuses its transfer: the batch table's grid of
     // this scene holds the P2G of its current particles (the table's grid
     // and grid2 may be swapped relative to S.grid / grid2 here, by the
@@ -162,9 +169,8 @@ struct Solver {
     bool bprescat = false;
 };
 
-// Below this many particles the fused step sorts in full every step: the
-// radix sort of a small scene is a few launches and the update would add
-// more than it saves.
+// Below this many particles the update is one launch that needs no full sort
+// beside it (run_sort_small); from here on it is four, chosen on the device.
 #ifndef MPM_INC_MIN_PARTICLES
 #define MPM_INC_MIN_PARTICLES (int64_t(1) << 20)
 #endif
