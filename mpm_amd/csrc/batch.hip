@@ -81,8 +81,6 @@ struct Batch {
     SceneEntry* tab = nullptr;
     uint32_t* key_offsets = nullptr;
     int64_t* block_start = nullptr;
-    uint32_t* range_start = nullptr;  // tab_cap + 1 words: each member's first global slot, then ntot
-    std::vector<uint32_t> range_host;
     int tab_cap = 0;
     uint32_t *kin = nullptr, *iota = nullptr, *ka = nullptr, *va = nullptr, *kb = nullptr, *vb = nullptr;
     uint32_t *flags = nullptr, *items = nullptr, *item_scene = nullptr, *hist = nullptr, *scan_temp = nullptr;
@@ -183,11 +181,13 @@ int ensure_capacity(Batch& b, int64_t n) {
     (void)hipStreamSynchronize(b.st);
     int64_t c = std::max<int64_t>(std::max<int64_t>(n, 1), b.cap + b.cap / 2);
     uint32_t** bufs[] = {&b.kin, &b.iota, &b.ka, &b.va, &b.kb, &b.vb, &b.flags, &b.item_scene, &b.snap_k, &b.snap_p};
-    uint32_t** lists[] = {&b.moves.key, &b.moves.slot, &b.moves.pos, &b.moves.lb, &b.moves.del_b, &b.moves.ins_b};
-    uint32_t** tiles[] = {&b.moves.tcount, &b.moves.tnext};
+    uint32_t** lists[] = {&b.moves.key, &b.moves.slot, &b.moves.pos};
+    uint32_t** tiles[] = {&b.moves.tnet, &b.moves.tbase};
     for (auto pp : bufs) bfree(b, *(void**)pp);
     for (auto pp : lists) bfree(b, *(void**)pp);
     for (auto pp : tiles) bfree(b, *(void**)pp);
+    bfree(b, *(void**)&b.moves.gone);
+    bfree(b, *(void**)&b.moves.ins);
     bfree(b, *(void**)&b.items);
     bfree(b, *(void**)&b.hist);
     bfree(b, *(void**)&b.scan_temp);
@@ -198,10 +198,15 @@ int ensure_capacity(Batch& b, int64_t n) {
     b.move_cap = inc_sublist_cap(c);
     for (auto pp : lists)
         if ((rc = balloc(b, (void**)pp, (size_t)kMoveLists * b.move_cap * 4))) return rc;
+    const size_t nt = inc_tiles(c), gone = nt * (kIncTile / 32);
     for (auto pp : tiles)
-        if ((rc = balloc(b, (void**)pp, (size_t)2 * (inc_tiles(c) + 1) * 4))) return rc;
-    // the merge keeps the counts zero afterwards
-    HIP_TRY(hipMemsetAsync(b.moves.tcount, 0, (size_t)2 * (inc_tiles(c) + 1) * 4, b.st));
+        if ((rc = balloc(b, (void**)pp, nt * 4))) return rc;
+    if ((rc = balloc(b, (void**)&b.moves.gone, gone * 4))) return rc;
+    if ((rc = balloc(b, (void**)&b.moves.ins, nt * kIncBucket * sizeof(uint2)))) return rc;
+    // each step's sort leaves them zero
+    HIP_TRY(hipMemsetAsync(b.moves.gone, 0, gone * 4, b.st));
+    HIP_TRY(hipMemsetAsync(b.moves.tnet, 0, nt * 4, b.st));
+    HIP_TRY(hipMemsetAsync(b.moves.ins, 0, nt * kIncBucket * sizeof(uint2), b.st));
     if (!b.moves_dev && (rc = balloc(b, (void**)&b.moves_dev, sizeof(MoveList)))) return rc;
     if (!b.plan && (rc = balloc(b, (void**)&b.plan, kPlanWords * 4))) return rc;
     HIP_TRY(hipMemcpyAsync(b.moves_dev, &b.moves, sizeof(MoveList), hipMemcpyHostToDevice, b.st));
@@ -342,12 +347,10 @@ int relayout(Batch& b) {
         bfree(b, *(void**)&b.tab);
         bfree(b, *(void**)&b.key_offsets);
         bfree(b, *(void**)&b.block_start);
-        bfree(b, *(void**)&b.range_start);
         const int c = std::max(ns, std::max(16, b.tab_cap * 2));
         if ((rc = balloc(b, (void**)&b.tab, (size_t)c * sizeof(SceneEntry)))) return rc;
         if ((rc = balloc(b, (void**)&b.key_offsets, (size_t)c * 4))) return rc;
         if ((rc = balloc(b, (void**)&b.block_start, (size_t)(c + 1) * 8))) return rc;
-        if ((rc = balloc(b, (void**)&b.range_start, (size_t)(c + 1) * 4))) return rc;
         b.tab_cap = c;
     }
     if (ns > 0) {
@@ -355,12 +358,6 @@ int relayout(Batch& b) {
         HIP_TRY(hipMemcpyAsync(b.key_offsets, b.koff_host.data(), (size_t)ns * 4, hipMemcpyHostToDevice, b.st));
     }
     HIP_TRY(hipMemcpyAsync(b.block_start, b.bstart_host.data(), (size_t)(ns + 1) * 8, hipMemcpyHostToDevice, b.st));
-    b.range_host.resize((size_t)ns + 1);
-    for (int i = 0; i < ns; ++i) b.range_host[(size_t)i] = (uint32_t)b.tab_host[(size_t)i].pstart;
-    b.range_host[(size_t)ns] = (uint32_t)n;
-    HIP_TRY(hipMemcpyAsync(b.range_start, b.range_host.data(), (size_t)(ns + 1) * 4, hipMemcpyHostToDevice, b.st));
-    b.moves.range_start = b.range_start;
-    b.moves.nranges = (uint32_t)ns;
     launch_iota(b.iota, n, b.st);
     b.I = ItemsDev{};
     b.I.start = b.items;
@@ -483,7 +480,7 @@ void enqueue_step(Batch& b, bool fused, bool scattered, bool full_sort, bool ove
         launch_reorder_chunk(b.tab, b.slot_scene, sel ? b.vb : b.va, b.chunk_bounds, b.chunk_rr, b.nchunks,
                              b.chunk_max, b.chunk_scratch, b.apic != 0, b.st);
     launch_items(b.I.sorted_keys, b.ntot, b.flags, b.scan_temp, b.items, b.counters, b.st, (uint32_t)b.tune.item_max,
-                 b.key_offsets, ns, b.item_scene, plan);
+                 b.key_offsets, ns, b.item_scene, plan, plan ? b.moves.tnet : nullptr);
     const SceneDev S0{};
     const ParticlesDev P0{};
     const int wgs = effective_wgs(b);

@@ -12,6 +12,7 @@ constexpr int kScanWG = 256;
 constexpr int kScanIPT = 4;
 constexpr int kScanTile = kScanWG * kScanIPT;
 
+template <int WG = kScanWG>  // threads of the workgroup
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* wave_sums, uint32_t& block_total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint32_t incl = v;
@@ -23,7 +24,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* w
     if (lane == 63) wave_sums[wave] = incl;
     __syncthreads();
     uint32_t pre = 0, tot = 0;
-    for (int w = 0; w < kScanWG / 64; ++w) {
+    for (int w = 0; w < WG / 64; ++w) {
         uint32_t s = wave_sums[w];
         if (w < wave) pre += s;
         tot += s;

@@ -527,7 +527,7 @@ void run_sort_incremental(Solver& s) {
     {
         Scope sc(h, "items");  // also resets the plan words for this step's G2P
         launch_items(s.I.sorted_keys, s.N, s.flags, s.scan_temp, s.items, s.counters, s.st, 0, nullptr, 0, nullptr,
-                     s.plan);
+                     s.plan, s.moves.tnet);
     }
     s.sort_valid = true;
 }
@@ -762,13 +762,17 @@ int build(Solver& s, HostState& H, int run_init) {
         if ((rc = dalloc(s, (void**)&s.plan, kPlanWords * 4))) return rc;
         HIP_TRY(hipMemsetAsync(s.plan, 0, kPlanWords * 4, s.st));  // snapshot not valid yet
         s.move_cap = inc_sublist_cap(s.N);
-        uint32_t** lists[] = {&s.moves.key, &s.moves.slot, &s.moves.pos, &s.moves.lb, &s.moves.del_b, &s.moves.ins_b};
-        for (auto pp : lists)
+        for (uint32_t** pp : {&s.moves.key, &s.moves.slot, &s.moves.pos})
             if ((rc = dalloc(s, (void**)pp, (size_t)kMoveLists * s.move_cap * 4))) return rc;
-        const size_t tw = (size_t)2 * (inc_tiles(s.N) + 1);
-        if ((rc = dalloc(s, (void**)&s.moves.tcount, tw * 4))) return rc;
-        HIP_TRY(hipMemsetAsync(s.moves.tcount, 0, tw * 4, s.st));  // the merge keeps them zero afterwards
-        if ((rc = dalloc(s, (void**)&s.moves.tnext, tw * 4))) return rc;
+        const size_t tiles = inc_tiles(s.N), gone = tiles * (kIncTile / 32);
+        if ((rc = dalloc(s, (void**)&s.moves.gone, gone * 4))) return rc;
+        if ((rc = dalloc(s, (void**)&s.moves.tnet, tiles * 4))) return rc;
+        // each step's sort leaves them zero
+        HIP_TRY(hipMemsetAsync(s.moves.gone, 0, gone * 4, s.st));
+        HIP_TRY(hipMemsetAsync(s.moves.tnet, 0, tiles * 4, s.st));
+        if ((rc = dalloc(s, (void**)&s.moves.tbase, tiles * 4))) return rc;
+        if ((rc = dalloc(s, (void**)&s.moves.ins, tiles * kIncBucket * sizeof(uint2)))) return rc;
+        HIP_TRY(hipMemsetAsync(s.moves.ins, 0, tiles * kIncBucket * sizeof(uint2), s.st));
         if ((rc = dalloc(s, (void**)&s.moves_dev, sizeof(MoveList)))) return rc;
         HIP_TRY(hipMemcpyAsync(s.plan + kPlanCap, &s.move_cap, 4, hipMemcpyHostToDevice, s.st));
         HIP_TRY(hipHostMalloc((void**)&s.inc_host, 64, hipHostMallocDefault));

@@ -121,12 +121,13 @@ constexpr int kSmallLists = 16;   // of a scene below kIncMinParticles, each of 
 __host__ __device__ inline uint32_t small_list_cap(int64_t n) { return (uint32_t)((n + kSmallLists - 1) / kSmallLists); }
 constexpr int kMoveCountStride = 64;  // words between two sub-list counters
 constexpr int kIncTile = 2048;    // snapshot entries per merge workgroup
-constexpr int kIncStage = 512;    // removals or insertions a merge workgroup ranks in LDS
+constexpr int kIncStage = 512;    // insertions that a tile's bucket holds
+constexpr int kIncBucket = kIncStage + 16;  // its size: a line for the fill count, then the entries
 enum PlanWord {
     kPlanSnapOk = 1,    // the snapshot is the previous step's order
     kPlanIncSteps = 2,  // steps sorted by the update since creation
     kPlanCap = 3,       // capacity of one sub-list
-    kPlanOverflow = 4,  // a sub-list overflowed, or a snapshot tile drew more than kIncStage entries
+    kPlanOverflow = 4,  // a sub-list or a snapshot tile's bucket overflowed
     kPlanMoves = 5,     // entries of the move list of the last sort
     kPlanLists = 64,    // the sub-list counters: word kPlanLists + r * kMoveCountStride
     kPlanWords = kPlanLists + kMoveLists * kMoveCountStride
@@ -134,22 +135,17 @@ enum PlanWord {
 // The step's choice, read by every sort kernel: the update when the
 // snapshot is the previous step's order and nothing overflowed.  The words
 // change only between sorts (the transfer appends and may set the
-// overflow; the update's offsets kernel may set it before the radix
+// overflow; the update's routing may set it before the radix
 // kernels run; the item count of the step resets them).
 __host__ __device__ inline bool plan_incremental(const uint32_t* plan) {
     return plan[kPlanSnapOk] != 0u && plan[kPlanOverflow] == 0u;
 }
 struct MoveList {
     uint32_t *key, *slot, *pos;  // appended by the transfer: sub-list r at [r * cap, r * cap + count_r)
-    uint32_t* lb;                // per entry: its place among the snapshot
-    uint32_t* tcount;            // [2][tiles + 1]: removed positions, insertion places per snapshot tile (zero between steps)
-    uint32_t* tnext;             // [2][tiles + 1]: bucket cursors
-    uint32_t *del_b, *ins_b;     // removed positions, entry indices: bucketed by tile (capacity each)
-    // a batch (else nranges 0): range_start[0..nranges] the first global slot
-    // of each member and the total; a member's particles also fill exactly
-    // that range of sorted positions (its keys are one range of the key space)
-    const uint32_t* range_start;
-    uint32_t nranges;
+    uint32_t* gone;              // a bit per sorted position: taken out (zero between steps)
+    uint32_t* tnet;              // per snapshot tile: entries put in less taken out (zero between steps)
+    uint32_t* tbase;             // per snapshot tile: the sum of tnet before it (many tiles)
+    uint2* ins;                  // per snapshot tile kIncBucket words: the fill count (zero between steps), entries
 };
 
 // Work items of the block-tiled kernels: a contiguous run of sorted

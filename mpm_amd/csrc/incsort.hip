@@ -9,23 +9,30 @@
 //     snapshot) as it reads them;
 //   * G2P appends each particle whose new key differs from its old one to a
 //     list (new key, slot, old sorted position; kMoveLists sub-lists);
-//   * here every list entry finds its place among the snapshot (lb: the
-//     number of snapshot entries before it in (key, slot) order) by a binary
-//     search, and the removed positions and insertion places are bucketed
-//     by snapshot tile (counts, one scan, then an append per entry);
-//   * one pass over the snapshot tiles finishes the job: each workgroup
-//     ranks its tile's few removals and insertions in LDS and writes every
-//     unmoved entry at i - (removed before i) + (inserted at or before i)
-//     and every inserted entry at lb - (removed before lb) + (inserted
-//     before it).
+//   * k_inc_route marks every entry's old position as gone and puts the entry
+//     into the bucket of the snapshot tile its place lies in (a binary search
+//     over the tiles' first entries);
+//   * k_inc_merge, one workgroup per tile, finds the places in the tile,
+//     ranks the insertions that share one, and writes every unmoved entry at
+//     i - (removed before i) + (inserted at or before i) and every inserted
+//     entry at its place - (removed before it) + (inserted before it).
 // The result is bit-identical to a stable radix sort of the new keys.  The
 // device-side plan words pick this path or the full radix sort each step
 // (the other path's launches return at once): the full sort runs when the
-// list overflowed, a tile drew more entries than its merge stages, or the
+// list overflowed, a tile drew more entries than its bucket holds, or the
 // snapshot is not the previous step's (first step, state written, a
-// single scene's store reordered, a batch's layout changed).  The step's item count resets the words afterwards
-// (launch_items with plan).  Launch order within a step: launch_inc_prepare,
-// the radix sort (which reads the decision), launch_inc_merge.
+// single scene's store reordered, a batch's layout changed).  The step's item
+// count resets the words and the tile counts afterwards (launch_items with
+// plan).  Launch order within a step: launch_inc_prepare, the radix sort
+// (which reads the decision), launch_inc_merge.
+//
+// What bounds it: the merge's 16 bytes per particle; the routing is a chain
+// of dependent loads per entry, hidden behind the other entries.  Before,
+// every entry's place was searched in the whole snapshot, and the removals
+// and insertions were bucketed by counts, a scan in one workgroup and a second
+// pass (searches twice as long and two launches more).  Measured, the four
+// kernels before and the two now, us: 2.1M slab 38 -> 21, 8.4M slab 85 -> 45,
+// uneven batch of 12.6M 190 -> 90, served batch of 2.7M 114 -> 47.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -39,17 +46,6 @@ constexpr int kIncWG = 256;
 // (key, slot) order of two sort entries.
 __device__ __forceinline__ bool entry_less(uint32_t ka, uint32_t sa, uint32_t kb, uint32_t sb) {
     return ka < kb || (ka == kb && sa < sb);
-}
-
-// Number of entries of a[0..n) (ascending) that are < v.
-__device__ __forceinline__ uint32_t count_below(const uint32_t* a, uint32_t n, uint32_t v) {
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (a[mid] < v) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
 }
 
 __global__ void k_inc_set(uint32_t* plan, uint32_t snap_ok) {
@@ -71,146 +67,199 @@ __global__ void k_inc_set(uint32_t* plan, uint32_t snap_ok) {
     for (uint32_t q_ = (blockIdx.x / (uint32_t)kMoveLists) * kIncWG + threadIdx.x, j = base_ + q_; q_ < c_; \
          q_ += step_, j = base_ + q_)
 
-// Each list entry's place among the snapshot, by binary search (a chain
-// of dependent loads, the entries all in flight at once; in a batch within
-// the entry's member), and the tile counts of its old position and of its
-// place (zero on entry: the merge clears them after use).
-__global__ void __launch_bounds__(kIncWG) k_inc_locate(const uint32_t* __restrict__ plan, MoveList L,
-                                                       const uint32_t* __restrict__ snap_k,
-                                                       const uint32_t* __restrict__ snap_p, int64_t n,
-                                                       uint32_t tiles) {
+// Each list entry's old position marked, and the entry put into its tile's
+// bucket (its counter in a line of its own: atomics on one line wait for each
+// other).  The tiles' net change is counted apart, and only for the entries
+// that leave their tile, which about three in four do not: counted for all of
+// them in one word with the bucket's, a batch of 12.6M particles took 52 us
+// here, 31 now, the grid clear beside it.
+__global__ void __launch_bounds__(kIncWG) k_inc_route(uint32_t* __restrict__ plan, MoveList L,
+                                                      const uint32_t* __restrict__ snap_k,
+                                                      const uint32_t* __restrict__ snap_p, uint32_t tiles) {
     if (!plan_incremental(plan)) return;
     FOR_LIST_ENTRIES(plan, j) {
-        const uint32_t k = L.key[j], s = L.slot[j];
-        uint32_t lo = 0, hi = (uint32_t)n;  // the place lies in [lo, hi]
-        if (L.nranges) {  // a batch: within its member's range (a short search in a cached table first)
-            uint32_t a = 0, b = L.nranges;
-            while (b - a > 1) {
-                const uint32_t mid = (a + b) >> 1;
-                if (L.range_start[mid] <= s) a = mid;
-                else b = mid;
-            }
-            lo = L.range_start[a];
-            hi = L.range_start[a + 1];
+        const uint32_t k = L.key[j], s = L.slot[j], pos = L.pos[j];
+        atomicOr(&L.gone[pos >> 5], 1u << (pos & 31u));
+        uint32_t lo = 0, hi = tiles;  // the last tile whose first entry is not above (k, s)
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            const size_t i = (size_t)mid * kIncTile;
+            if (entry_less(k, s, snap_k[i], snap_p[i])) hi = mid;
+            else lo = mid;
         }
-        while (lo < hi) {
-            const uint32_t mid = lo + ((hi - lo) >> 1);
-            if (entry_less(snap_k[mid], snap_p[mid], k, s)) lo = mid + 1;
-            else hi = mid;
+        const uint32_t from = pos / (uint32_t)kIncTile;
+        if (from != lo) {
+            atomicAdd(&L.tnet[from], ~0u);
+            atomicAdd(&L.tnet[lo], 1u);
         }
-        L.lb[j] = lo;
-        atomicAdd(&L.tcount[L.pos[j] / (uint32_t)kIncTile], 1u);
-        atomicAdd(&L.tcount[tiles + 1u + lo / (uint32_t)kIncTile], 1u);
+        uint2* const bucket = L.ins + (size_t)lo * kIncBucket;
+        const uint32_t q = atomicAdd(&bucket->x, 1u);
+        if (q < (uint32_t)kIncStage) bucket[kIncBucket - kIncStage + q] = uint2{k, s};
+        else plan[kPlanOverflow] = 1u;
     }
 }
 
-// Bucket offsets: exclusive scans of the two count arrays (tiles + 1
-// entries each) into the bucket cursors, by one workgroup per array (each
-// thread a run of consecutive counts); a tile with more entries than the
-// merge stages sends this step to the full sort.
-__global__ void __launch_bounds__(kScanWG) k_inc_offsets(uint32_t* __restrict__ plan, MoveList L, uint32_t tiles) {
+// The net change of the tiles before each tile, by one workgroup: for more
+// than kSumTiles tiles (below, the merge's workgroups add up the tiles before
+// them themselves: one launch less, at most 16 loads a thread).
+constexpr uint32_t kSumTiles = 8192;
+__global__ void __launch_bounds__(kScanWG) k_inc_offsets(const uint32_t* __restrict__ plan, MoveList L,
+                                                         uint32_t tiles) {
     if (!plan_incremental(plan)) return;
     __shared__ uint32_t ws[kScanWG / 64];
-    const uint32_t m = tiles + 1u;
-    const uint32_t* const cnt = L.tcount + (size_t)blockIdx.x * m;
-    uint32_t* const cur = L.tnext + (size_t)blockIdx.x * m;
-    const uint32_t per = (m + kScanWG - 1) / kScanWG;
-    const uint32_t t0 = threadIdx.x * per < m ? threadIdx.x * per : m;
-    const uint32_t t1 = t0 + per < m ? t0 + per : m;
-    uint32_t sum = 0;
-    bool over = false;
-    for (uint32_t t = t0; t < t1; ++t) {
-        const uint32_t v = cnt[t];
-        over = over || v > (uint32_t)kIncStage;
-        sum += v;
-    }
-    uint32_t tot;
-    uint32_t run = block_exclusive_scan(sum, ws, tot);
-    for (uint32_t t = t0; t < t1; ++t) {
-        cur[t] = run;
-        run += cnt[t];
-    }
-    if (over) plan[kPlanOverflow] = 1u;
-}
-
-// Each entry's old position and entry index appended to the buckets of
-// their tiles (the order inside a bucket is arbitrary: the merge ranks it).
-__global__ void __launch_bounds__(kIncWG) k_inc_bucket(const uint32_t* __restrict__ plan, MoveList L,
-                                                       uint32_t tiles) {
-    if (!plan_incremental(plan)) return;
-    FOR_LIST_ENTRIES(plan, j) {
-        const uint32_t pos = L.pos[j], lb = L.lb[j];
-        L.del_b[atomicAdd(&L.tnext[pos / (uint32_t)kIncTile], 1u)] = pos;
-        L.ins_b[atomicAdd(&L.tnext[tiles + 1u + lb / (uint32_t)kIncTile], 1u)] = j;
-    }
-}
-
-// One snapshot tile [i0, i1) per workgroup (the last one, past n when n is
-// a multiple of the tile, takes the insertions at n); it also zeroes the
-// tile's counts, also on a step the update does not run (after an overflow
-// the counts are left over).  After the bucketing
-// the cursors sit at the end of each bucket, so a bucket starts at
-// cursor - count.  Removed positions are distinct and list entries have
-// distinct (key, slot), so ranking by counting gives each its own place.
-__global__ void __launch_bounds__(kIncWG) k_inc_merge(const uint32_t* __restrict__ plan, MoveList L,
-                                                      const uint32_t* __restrict__ snap_k,
-                                                      const uint32_t* __restrict__ snap_p, int64_t n, uint32_t tiles,
-                                                      uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_p) {
-    const uint32_t t = blockIdx.x;
-    if (!plan_incremental(plan)) {  // an overflow after the counting: clear them for the next step
-        if (threadIdx.x == 0) {
-            L.tcount[t] = 0u;
-            L.tcount[tiles + 1u + t] = 0u;
+    uint32_t before = 0;
+    for (uint32_t t0 = 0; t0 < tiles; t0 += kScanTile) {
+        uint32_t v[kScanIPT], sum = 0;
+#pragma unroll
+        for (int r = 0; r < kScanIPT; ++r) {
+            const uint32_t t = t0 + threadIdx.x * kScanIPT + r;
+            v[r] = t < tiles ? L.tnet[t] : 0u;
+            sum += v[r];
         }
+        uint32_t tot;
+        uint32_t run = before + block_exclusive_scan(sum, ws, tot);
+#pragma unroll
+        for (int r = 0; r < kScanIPT; ++r) {
+            const uint32_t t = t0 + threadIdx.x * kScanIPT + r;
+            if (t < tiles) L.tbase[t] = run;
+            run += v[r];
+        }
+        before += tot;
+    }
+}
+
+constexpr int kTileIPT = 4;  // entries per thread of the tiles below
+
+// Number of tile entries below (key, slot).
+__device__ __forceinline__ uint32_t place_in_tile(const uint32_t* sk, const uint32_t* sp, uint32_t cnt, uint32_t k,
+                                                  uint32_t s) {
+    uint32_t lo = 0, hi = cnt;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (entry_less(sk[mid], sp[mid], k, s)) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Number of entries of a[0..n) (ascending) that are < v.
+__device__ __forceinline__ uint32_t count_below(const uint32_t* a, uint32_t n, uint32_t v) {
+    uint32_t lo = 0, hi = n;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (a[mid] < v) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// One snapshot tile per workgroup, its entries in registers (and in LDS for
+// the search of the places); it also clears the tile's marks and bucket
+// for the next step (on a step that the update does not run too: after an overflow some
+// are left).  The few insertions are ranked by counting, so that an entry
+// finds its shift by one popcount and a search among the places.  tbase:
+// where k_inc_offsets has run, else null.
+__global__ void __launch_bounds__(kIncTile / kTileIPT) k_inc_merge(const uint32_t* __restrict__ plan, MoveList L,
+                                                                   const uint32_t* __restrict__ snap_k,
+                                                                   const uint32_t* __restrict__ snap_p, uint32_t n,
+                                                                   const uint32_t* __restrict__ tbase,
+                                                                   uint32_t* __restrict__ out_k,
+                                                                   uint32_t* __restrict__ out_p) {
+    constexpr int WG = kIncTile / kTileIPT, WORDS = kIncTile / 32;
+    static_assert(WORDS == 64, "the marks of a tile are scanned by one wave");
+    __shared__ uint32_t sk[kIncTile], sp[kIncTile];
+    __shared__ uint32_t gone[WORDS + 1], gone_before[WORDS + 1];  // one more: the end of a full tile
+    __shared__ uint32_t mk[kIncStage], ms[kIncStage], sorted[kIncStage];  // insertions; their places, ascending
+    __shared__ uint32_t ws[WG / 64];
+    const uint32_t t = blockIdx.x, tid = threadIdx.x;
+    const uint32_t i0 = t * kIncTile, cnt = n - i0 < kIncTile ? n - i0 : kIncTile;
+    uint32_t* const marks = L.gone + (size_t)t * WORDS;
+    uint2* const bucket = L.ins + (size_t)t * kIncBucket;
+    if (!plan_incremental(plan)) {
+        if (tid < WORDS) marks[tid] = 0u;
+        if (tid == 0) bucket->x = 0u;
         return;
     }
-    __shared__ uint32_t dr[kIncStage], sdel[kIncStage];              // removed positions: as bucketed, ascending
-    __shared__ uint32_t ir[kIncStage], ik[kIncStage], is[kIncStage];  // insertions: place, key, slot
-    __shared__ uint32_t slb[kIncStage];                                // insertion places, ascending
-    const int64_t i0 = (int64_t)t * kIncTile;
-    const int64_t i1 = i0 + kIncTile < n ? i0 + kIncTile : n;
-    const uint32_t dc = L.tcount[t], rc = L.tcount[tiles + 1u + t];  // <= kIncStage (else overflow)
-    const uint32_t d0 = L.tnext[t] - dc, r0 = L.tnext[tiles + 1u + t] - rc;
-    for (uint32_t q = threadIdx.x; q < dc; q += kIncWG) dr[q] = L.del_b[d0 + q];
-    for (uint32_t q = threadIdx.x; q < rc; q += kIncWG) {
-        const uint32_t j = L.ins_b[r0 + q];
-        ir[q] = L.lb[j];
-        ik[q] = L.key[j];
-        is[q] = L.slot[j];
+    const uint32_t drawn = bucket->x;  // at most kIncStage (else overflow)
+    const uint32_t nm = drawn < (uint32_t)kIncStage ? drawn : (uint32_t)kIncStage;
+    uint32_t key[kTileIPT], slot[kTileIPT];
+#pragma unroll
+    for (int r = 0; r < kTileIPT; ++r) {
+        const uint32_t i = tid + r * WG, ic = i < cnt ? i : 0u;
+        key[r] = snap_k[i0 + ic];
+        slot[r] = snap_p[i0 + ic];
     }
-    __syncthreads();  // every thread has read the counts
-    if (threadIdx.x == 0) {  // zero for the next step's counting
-        L.tcount[t] = 0u;
-        L.tcount[tiles + 1u + t] = 0u;
+    for (uint32_t q = tid; q < nm; q += WG) {
+        const uint2 e = bucket[kIncBucket - kIncStage + q];
+        mk[q] = e.x;
+        ms[q] = e.y;
     }
-    for (uint32_t q = threadIdx.x; q < dc; q += kIncWG) {
-        const uint32_t v = dr[q];
-        uint32_t r = 0;
-        for (uint32_t x = 0; x < dc; ++x) r += dr[x] < v ? 1u : 0u;
-        sdel[r] = v;
+    if (tid < WORDS) {  // one wave
+        const uint32_t w = marks[tid];
+        marks[tid] = 0u;
+        uint32_t incl = (uint32_t)__popc(w);
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t up = __shfl_up(incl, off, 64);
+            if ((int)tid >= off) incl += up;
+        }
+        gone[tid] = w;
+        gone_before[tid] = incl - (uint32_t)__popc(w);
+        if (tid == WORDS - 1) {
+            gone[WORDS] = 0u;
+            gone_before[WORDS] = incl;
+        }
     }
-    __syncthreads();
-    for (uint32_t q = threadIdx.x; q < rc; q += kIncWG) {
-        const uint32_t k = ik[q], s = is[q], lb = ir[q];
-        uint32_t r = 0;  // (key, slot) order is also the order of the places
-        for (uint32_t x = 0; x < rc; ++x) r += entry_less(ik[x], is[x], k, s) ? 1u : 0u;
-        slb[r] = lb;
-        const uint32_t dst = lb - (d0 + count_below(sdel, dc, lb)) + r0 + r;
-        if ((int64_t)dst < n) {  // always, for a list that matches the snapshot
+    if (nm) {
+#pragma unroll
+        for (int r = 0; r < kTileIPT; ++r) {
+            sk[tid + r * WG] = key[r];
+            sp[tid + r * WG] = slot[r];
+        }
+    }
+    uint32_t shift = 0;
+    if (tbase) {
+        shift = tbase[t];
+        __syncthreads();
+    } else {
+        // eight loads in flight at a time: the sum is a latency, not work
+        uint32_t part = 0;
+        for (uint32_t q = tid; q < t; q += 8 * WG) {
+            uint32_t c[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) c[u] = L.tnet[q + u * WG < t ? q + u * WG : t];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u)
+                if (q + u * WG < t) part += c[u];
+        }
+        block_exclusive_scan<WG>(part, ws, shift);
+    }
+    if (tid == 0) bucket->x = 0u;  // every thread has read it
+    const uint32_t base = i0 + shift;
+    auto removed = [&](uint32_t i) -> uint32_t {  // before position i of the tile
+        return gone_before[i >> 5] + (uint32_t)__popc(gone[i >> 5] & ((1u << (i & 31u)) - 1u));
+    };
+    for (uint32_t q = tid; q < nm; q += WG) {
+        const uint32_t k = mk[q], s = ms[q];
+        const uint32_t l = place_in_tile(sk, sp, cnt, k, s);
+        uint32_t rank = 0;  // (key, slot) order is also the order of the places
+        for (uint32_t x = 0; x < nm; ++x) rank += entry_less(mk[x], ms[x], k, s) ? 1u : 0u;
+        sorted[rank] = l;
+        const uint32_t dst = base + l - removed(l) + rank;
+        if (dst < n) {  // always, for a list that matches the snapshot
             out_k[dst] = k;
             out_p[dst] = s;
         }
     }
-    __syncthreads();
-    // consecutive lanes take consecutive entries: loads and (shifted) stores stay contiguous
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += kIncWG) {
-        const uint32_t iu = (uint32_t)i;
-        const uint32_t dl = count_below(sdel, dc, iu);
-        if (dl < dc && sdel[dl] == iu) continue;  // moved
-        const uint32_t dst = iu - (d0 + dl) + r0 + count_below(slb, rc, iu + 1u);  // places <= i
-        if ((int64_t)dst < n) {
-            out_k[dst] = snap_k[i];
-            out_p[dst] = snap_p[i];
+    if (nm) __syncthreads();  // uniform
+#pragma unroll
+    for (int r = 0; r < kTileIPT; ++r) {
+        const uint32_t i = tid + r * WG;
+        if (i >= cnt || ((gone[i >> 5] >> (i & 31u)) & 1u)) continue;
+        const uint32_t dst = base + i - removed(i) + count_below(sorted, nm, i + 1u);  // places <= i
+        if (dst < n) {
+            out_k[dst] = key[r];
+            out_p[dst] = slot[r];
         }
     }
 }
@@ -228,18 +277,80 @@ __global__ void __launch_bounds__(kIncWG) k_inc_merge(const uint32_t* __restrict
 // L2); the host takes the radix sort instead where that is the larger (see
 // run_sort_small).  Measured at 16,384 particles: six radix launches of 41 us
 // and their gaps and a grid clear of 5 us before, one of 8.6 us for both now.
-constexpr int kMatch = 512;  // of a tile's insertions, those kept in LDS
-
-// Number of tile entries below (key, slot).
-__device__ __forceinline__ uint32_t place_in_tile(const uint32_t* sk, const uint32_t* sp, uint32_t cnt, uint32_t k,
-                                                  uint32_t s) {
-    uint32_t lo = 0, hi = cnt;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (entry_less(sk[mid], sp[mid], k, s)) lo = mid + 1;
-        else hi = mid;
+// A tile of the last order in LDS, the positions taken out of it and what is
+// put into it.
+constexpr int kMatch = 512;  // insertions kept in LDS
+template <int TILE>
+struct TileLds {
+    uint32_t sk[TILE], sp[TILE];
+    uint32_t ins[TILE + 1];     // insertions at each place of the tile (TILE: after its last entry)
+    uint32_t before[TILE + 1];  // removals (low 12 bits) and insertions before each place
+    uint32_t gone[TILE / 32];   // removed positions
+    uint32_t mk[kMatch], ms[kMatch], place[kMatch];  // insertions and their places
+    uint32_t nmatch, ws[TILE / kTileIPT / 64];
+    // first place in the new order of what is inserted at place l; base: of the tile
+    __device__ __forceinline__ uint32_t bucket(uint32_t base, uint32_t l) const {
+        return base + l - (before[l] & 4095u) + (before[l] >> 12);
     }
-    return lo;
+};
+
+// Counts the nm insertions in T.mk/T.ms into T.ins, scans the places and
+// writes the tile's unmoved entries; base: where the tile begins in the new
+// order.  Call it after a barrier; ends with T complete for every thread.
+template <int TILE>
+__device__ __forceinline__ void update_unmoved(TileLds<TILE>& T, uint32_t cnt, uint32_t nm, uint32_t n, uint32_t base,
+                                               uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_p) {
+    constexpr int IPT = kTileIPT, WG = TILE / IPT;
+    static_assert(TILE <= 2048, "removals of a tile take 12 bits of `before`");
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t q = tid; q < nm; q += WG) {
+        T.place[q] = place_in_tile(T.sk, T.sp, cnt, T.mk[q], T.ms[q]);
+        atomicAdd(&T.ins[T.place[q]], 1u);
+    }
+    __syncthreads();
+    // thread tid scans places IPT * tid ..
+    uint32_t d[IPT], c[IPT];
+    uint32_t ds = 0, is = 0, dsum, isum;
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const uint32_t i = tid * IPT + r;
+        d[r] = ds;
+        c[r] = is;
+        ds += (T.gone[i >> 5] >> (i & 31u)) & 1u;
+        is += T.ins[i];
+    }
+    const uint32_t dpre = block_exclusive_scan<WG>(ds, T.ws, dsum);
+    const uint32_t ipre = block_exclusive_scan<WG>(is, T.ws, isum);
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) T.before[tid * IPT + r] = (dpre + d[r]) | ((ipre + c[r]) << 12);
+    if (tid == 0) T.before[TILE] = dsum | (isum << 12);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const uint32_t i = tid + r * WG;
+        if (i >= cnt || ((T.gone[i >> 5] >> (i & 31u)) & 1u)) continue;
+        const uint32_t dst = T.bucket(base, i) + T.ins[i];
+        if (dst < n) {  // always, for a list that matches the snapshot
+            out_k[dst] = T.sk[i];
+            out_p[dst] = T.sp[i];
+        }
+    }
+}
+// The nm insertions themselves, ranked among those at the same place.
+template <int TILE>
+__device__ __forceinline__ void update_inserted(const TileLds<TILE>& T, uint32_t nm, uint32_t n, uint32_t base,
+                                                uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_p) {
+    for (uint32_t q = threadIdx.x; q < nm; q += TILE / kTileIPT) {
+        const uint32_t k = T.mk[q], s = T.ms[q], l = T.place[q];
+        uint32_t rank = 0;
+        if (T.ins[l] > 1u)
+            for (uint32_t x = 0; x < nm; ++x) rank += T.place[x] == l && entry_less(T.mk[x], T.ms[x], k, s) ? 1u : 0u;
+        const uint32_t dst = T.bucket(base, l) + rank;
+        if (dst < n) {
+            out_k[dst] = k;
+            out_p[dst] = s;
+        }
+    }
 }
 
 // Clear of the touched blocks of a grid, 8 consecutive blocks per wave.
@@ -269,14 +380,10 @@ __global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restri
         clear_blocks(C, (int64_t)(blockIdx.x - tiles) * (kIncWG / 64) + (threadIdx.x >> 6));
         return;
     }
-    constexpr int TILE = kUpdateTile, IPT = TILE / kIncWG;
-    __shared__ uint32_t sk[TILE], sp[TILE];
-    __shared__ uint32_t ins[TILE + 1];        // insertions at each place of the tile (TILE: after its last entry)
-    __shared__ uint32_t before[TILE + 1];     // removals (low 11 bits) and insertions before each place
-    __shared__ uint32_t gone[TILE / 32];      // removed positions
-    __shared__ uint32_t mk[kMatch], ms[kMatch], place[kMatch];  // the tile's insertions and their places
-    __shared__ uint32_t nmatch, ws[kIncWG / 64];
-    static_assert(TILE <= 1024, "removals of a tile take 11 bits of `before`");
+    constexpr int TILE = kUpdateTile, IPT = kTileIPT;
+    static_assert(TILE == kIncWG * IPT);
+    __shared__ TileLds<TILE> T;
+    uint32_t (&sk)[TILE] = T.sk, (&sp)[TILE] = T.sp, (&ins)[TILE + 1] = T.ins;
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
     const uint32_t i0 = t * TILE, cnt = n - i0 < TILE ? n - i0 : TILE;
     const bool last = t + 1 == tiles;
@@ -289,10 +396,10 @@ __global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restri
         }
         ins[i] = 0u;
     }
-    if (tid < TILE / 32) gone[tid] = 0u;
+    if (tid < TILE / 32) T.gone[tid] = 0u;
     if (tid == 0) {
         ins[TILE] = 0u;
-        nmatch = 0u;
+        T.nmatch = 0u;
     }
     const uint32_t nk = last ? 0u : snap_k[i0 + TILE], np = last ? 0u : snap_p[i0 + TILE];
     __syncthreads();
@@ -340,81 +447,48 @@ __global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restri
     uint32_t db = 0, ib = 0;
     for_list([&](uint32_t k, uint32_t s, uint32_t pos) {
         if (pos < i0) ++db;
-        else if (pos - i0 < cnt) atomicOr(&gone[(pos - i0) >> 5], 1u << ((pos - i0) & 31u));
+        else if (pos - i0 < cnt) atomicOr(&T.gone[(pos - i0) >> 5], 1u << ((pos - i0) & 31u));
         const int w = side(k, s);
         if (w < 0) ++ib;
         if (w == 0) {
-            const uint32_t q = atomicAdd(&nmatch, 1u);
+            const uint32_t q = atomicAdd(&T.nmatch, 1u);
             if (q < kMatch) {
-                mk[q] = k;
-                ms[q] = s;
+                T.mk[q] = k;
+                T.ms[q] = s;
             } else {
                 atomicAdd(&ins[place_in_tile(sk, sp, cnt, k, s)], 1u);
             }
         }
     });
     __syncthreads();
-    const uint32_t nm = nmatch;
-    for (uint32_t q = tid; q < (nm < kMatch ? nm : kMatch); q += kIncWG) {
-        place[q] = place_in_tile(sk, sp, cnt, mk[q], ms[q]);
-        atomicAdd(&ins[place[q]], 1u);
-    }
-    __syncthreads();
-    uint32_t dtot, itot, dsum, isum;
-    block_exclusive_scan(db, ws, dtot);
-    block_exclusive_scan(ib, ws, itot);
-    // thread tid scans places IPT * tid ..
-    uint32_t d[IPT], c[IPT];
-    uint32_t ds = 0, is = 0;
-#pragma unroll
-    for (int r = 0; r < IPT; ++r) {
-        const uint32_t i = tid * IPT + r;
-        d[r] = ds;
-        c[r] = is;
-        ds += (gone[i >> 5] >> (i & 31u)) & 1u;
-        is += ins[i];
-    }
-    const uint32_t dpre = block_exclusive_scan(ds, ws, dsum);
-    const uint32_t ipre = block_exclusive_scan(is, ws, isum);
-#pragma unroll
-    for (int r = 0; r < IPT; ++r) before[tid * IPT + r] = (dpre + d[r]) | ((ipre + c[r]) << 11);
-    if (tid == 0) before[TILE] = dsum | (isum << 11);
-    __syncthreads();
+    const uint32_t nm = T.nmatch;
+    uint32_t dtot, itot;
+    block_exclusive_scan(db, T.ws, dtot);
+    block_exclusive_scan(ib, T.ws, itot);
     const uint32_t base = i0 - dtot + itot;
-    // first place in the new order of what is inserted at place l
-    auto bucket = [&](uint32_t l) -> uint32_t { return base + l - (before[l] & 2047u) + (before[l] >> 11); };
-#pragma unroll
-    for (int r = 0; r < IPT; ++r) {
-        const uint32_t i = tid + r * kIncWG;
-        if (i >= cnt || ((gone[i >> 5] >> (i & 31u)) & 1u)) continue;
-        const uint32_t dst = bucket(i) + ins[i];
-        if (dst < n) {  // always, for a list that matches the snapshot
-            out_k[dst] = sk[i];
-            out_p[dst] = sp[i];
-        }
+    update_unmoved(T, cnt, nm < kMatch ? nm : kMatch, n, base, out_k, out_p);
+    if (nm <= (uint32_t)kMatch) {  // uniform
+        update_inserted(T, nm, n, base, out_k, out_p);
+        return;
     }
-    if (nm == 0u) return;  // uniform
-    __syncthreads();       // sk is free: from here on the bucket cursors
+    // more: put into scratch in arbitrary order, then ranked.  Their places
+    // need sk again, which holds the cursors, so they are found in the
+    // snapshot in memory
+    __syncthreads();
     uint32_t* const cur = sk;
 #pragma unroll
     for (int r = 0; r < IPT; ++r) cur[tid + r * kIncWG] = 0u;
-    // the places were found with sk; entries beyond kMatch need it again, so
-    // their place is found in the snapshot in memory
     __shared__ uint32_t cur_last;
     if (tid == 0) cur_last = 0u;
     __syncthreads();
     auto for_matches = [&](auto&& fn) {
-        if (nm <= kMatch) {
-            for (uint32_t q = tid; q < nm; q += kIncWG) fn(mk[q], ms[q], place[q]);
-        } else {
-            for_list([&](uint32_t k, uint32_t s, uint32_t) {
-                if (side(k, s) == 0) fn(k, s, place_in_tile(snap_k + i0, snap_p + i0, cnt, k, s));
-            });
-        }
+        for_list([&](uint32_t k, uint32_t s, uint32_t) {
+            if (side(k, s) == 0) fn(k, s, place_in_tile(snap_k + i0, snap_p + i0, cnt, k, s));
+        });
     };
     for_matches([&](uint32_t k, uint32_t s, uint32_t l) {
         const uint32_t u = atomicAdd(l < TILE ? &cur[l] : &cur_last, 1u);
-        const uint32_t dst = bucket(l) + u;
+        const uint32_t dst = T.bucket(base, l) + u;
         if (dst >= n) return;
         uint32_t* const ok = ins[l] == 1u ? out_k : tmp_k;
         uint32_t* const op = ins[l] == 1u ? out_p : tmp_p;
@@ -423,7 +497,7 @@ __global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restri
     });
     __syncthreads();
     for_matches([&](uint32_t k, uint32_t s, uint32_t l) {
-        const uint32_t c0 = ins[l], b0 = bucket(l);
+        const uint32_t c0 = ins[l], b0 = T.bucket(base, l);
         if (c0 == 1u || b0 + c0 > n) return;
         uint32_t rank = 0;
         for (uint32_t u = 0; u < c0; ++u) rank += entry_less(tmp_k[b0 + u], tmp_p[b0 + u], k, s) ? 1u : 0u;
@@ -451,7 +525,7 @@ void launch_sort_update(const uint32_t* plan, const MoveList& L, const uint32_t*
                        tiles, out_k, out_p, tmp_k, tmp_p, clear);
 }
 
-uint32_t inc_tiles(int64_t n) { return (uint32_t)(n / kIncTile + 1); }
+uint32_t inc_tiles(int64_t n) { return (uint32_t)((n + kIncTile - 1) / kIncTile); }
 
 void launch_inc_set(uint32_t* plan, uint32_t snap_ok, hipStream_t st) {
     hipLaunchKernelGGL(k_inc_set, dim3(1), dim3(64), 0, st, plan, snap_ok);
@@ -459,18 +533,20 @@ void launch_inc_set(uint32_t* plan, uint32_t snap_ok, hipStream_t st) {
 
 void launch_inc_prepare(uint32_t* plan, const MoveList& L, const uint32_t* snap_k, const uint32_t* snap_p, int64_t n,
                         hipStream_t st) {
-    const uint32_t tiles = inc_tiles(n);
+    if (n <= 0) return;
     // 16 workgroups per sub-list
-    hipLaunchKernelGGL(k_inc_locate, dim3(16 * kMoveLists), dim3(kIncWG), 0, st, plan, L, snap_k, snap_p, n, tiles);
-    hipLaunchKernelGGL(k_inc_offsets, dim3(2), dim3(kScanWG), 0, st, plan, L, tiles);
+    hipLaunchKernelGGL(k_inc_route, dim3(16 * kMoveLists), dim3(kIncWG), 0, st, plan, L, snap_k, snap_p,
+                       inc_tiles(n));
 }
 
 void launch_inc_merge(const uint32_t* plan, const MoveList& L, const uint32_t* snap_k, const uint32_t* snap_p,
                       int64_t n, uint32_t* out_k, uint32_t* out_p, hipStream_t st) {
+    if (n <= 0) return;
     const uint32_t tiles = inc_tiles(n);
-    hipLaunchKernelGGL(k_inc_bucket, dim3(16 * kMoveLists), dim3(kIncWG), 0, st, plan, L, tiles);
-    hipLaunchKernelGGL(k_inc_merge, dim3(tiles), dim3(kIncWG), 0, st, plan, L, snap_k, snap_p, n, tiles, out_k,
-                       out_p);
+    const bool scanned = tiles > kSumTiles;
+    if (scanned) hipLaunchKernelGGL(k_inc_offsets, dim3(1), dim3(kScanWG), 0, st, plan, L, tiles);
+    hipLaunchKernelGGL(k_inc_merge, dim3(tiles), dim3(kIncTile / kTileIPT), 0, st, plan, L, snap_k, snap_p,
+                       (uint32_t)n, scanned ? (const uint32_t*)L.tbase : nullptr, out_k, out_p);
 }
 
 }  // namespace mpm

@@ -62,9 +62,8 @@ void launch_sort_update(const uint32_t* plan, const MoveList& L, const uint32_t*
                         const GridClear& clear, hipStream_t st);
 void launch_update_init(uint32_t* plan, MoveList* dev, const MoveList& L, hipStream_t st);  // empty list, no snapshot
 constexpr int kUpdateTile = 1024;  // snapshot entries per workgroup of it
-// Sizes of the update's buffers for n particles: snapshot tiles (the tile
-// arrays hold 2 * (tiles + 1) words each) and the capacity of one sub-list
-// (the list arrays hold kMoveLists times that).
+// Sizes of the update's buffers for n particles: snapshot tiles and the
+// capacity of one sub-list (the list arrays hold kMoveLists times that).
 uint32_t inc_tiles(int64_t n);
 inline uint32_t inc_sublist_cap(int64_t n) {
     const int64_t cap = n / 8 > kMoveMin ? n / 8 : kMoveMin;
@@ -83,10 +82,13 @@ void launch_iota(uint32_t* p, int64_t n, hipStream_t st);
 // items[n..2n) their key blocks (so items holds 2n words).  item_max = 0
 // picks a multiple of 64 up to kItemMax from n (about four items per compute
 // unit for small n).  For a batch, key_offsets[nscenes] (ascending) gives
-// each item's scene in item_scene.
+// each item's scene in item_scene.  plan: the incremental sort's words, reset
+// for the step's G2P, with the tiles' net counts, zeroed (null: a small
+// scene's update has none).
 void launch_items(const uint32_t* sorted_keys, int64_t n, uint32_t* flags, uint32_t* scan_temp, uint32_t* items,
                   uint32_t* item_count, hipStream_t st, uint32_t item_max = 0, const uint32_t* key_offsets = nullptr,
-                  int nscenes = 0, uint32_t* item_scene = nullptr, uint32_t* plan = nullptr);
+                  int nscenes = 0, uint32_t* item_scene = nullptr, uint32_t* plan = nullptr,
+                  uint32_t* tile_net = nullptr);
 
 // grid_wgs: persistent workgroups; 0 = one resident round (occupancy of the
 // kernel instance x compute units).
