@@ -2906,66 +2906,77 @@ void launch_count_escaped(const uint32_t* sorted_keys, int64_t n, uint32_t escap
 // particles with a non-finite position or velocity component, and the
 // particles whose next key is the scene's escape key (stencil outside the
 // grid).  keys: the global sort input the last G2P wrote (key offset +
-// cell key per slot), so a slot's scene is the last whose key offset is <=
-// its key.  out: 3 words per scene, zeroed by the caller.
+// cell key per slot).  out: 3 words per scene, zeroed by the caller.
+//
+// A workgroup takes a contiguous run of slots, scene by scene, and adds to a
+// scene's words once: they share a few cache lines, where atomics wait for
+// each other (one per wave of 64 slots: 279 us for 24 scenes of 2.6M
+// particles, 25 us now, where the 28 bytes per particle take 14).
 __global__ void __launch_bounds__(256) k_batch_health(const SceneEntry* __restrict__ tab,
                                                       const uint32_t* __restrict__ key_offsets, int ns, int64_t ntot,
-                                                      const uint32_t* __restrict__ keys, uint32_t* __restrict__ out) {
-    const int lane = threadIdx.x & 63;
-    for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x; i0 < ntot; i0 += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t i = i0 + threadIdx.x;
-        const bool act = i < ntot;
-        int sc = 0;
-        uint32_t q = 0, bad = 0, esc = 0;
-        if (act) {
-            const uint32_t key = keys[i];
-            int lo = 0, hi = ns - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (key_offsets[mid] <= key) lo = mid;
-                else hi = mid - 1;
-            }
-            sc = lo;
-            const int64_t p = i - tab[sc].pstart;
-            const int64_t N = tab[sc].P.n;
-            const float* x = tab[sc].P.x;
-            const float* v = tab[sc].P.v;
+                                                      int64_t per, const uint32_t* __restrict__ keys,
+                                                      uint32_t* __restrict__ out) {
+    __shared__ uint32_t part[4][3];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int64_t i0 = (int64_t)blockIdx.x * per;
+    const int64_t i1 = i0 + per < ntot ? i0 + per : ntot;
+    int sc = 0, hi = ns - 1;
+    while (sc < hi) {  // the last scene whose first slot is <= i0
+        const int mid = (sc + hi + 1) >> 1;
+        if (tab[mid].pstart <= i0) sc = mid;
+        else hi = mid - 1;
+    }
+    for (; i0 < i1 && sc < ns; ++sc) {
+        const int64_t base = tab[sc].pstart, N = tab[sc].P.n;
+        const int64_t end = base + N < i1 ? base + N : i1;
+        if (end <= i0) continue;  // an empty scene
+        const uint32_t escape = key_offsets[sc] + tab[sc].S.escape_key;
+        const auto x = tab[sc].P.x, v = tab[sc].P.v;
+        uint32_t m = 0, nb = 0, ne = 0;
+        for (int64_t i = i0 + threadIdx.x; i < end; i += 256) {
+            const int64_t p = i - base;
             const float a = v[p], b = v[N + p], c = v[2 * N + p];
             const float x0 = x[p], x1 = x[N + p], x2 = x[2 * N + p];
             const float sq = (a * a + b * b) + c * c;
-            q = __float_as_uint(sq) & 0x7FFFFFFFu;  // |v|^2 >= 0; a NaN keeps its payload above +inf
-            bad = (isfinite(a) && isfinite(b) && isfinite(c) && isfinite(x0) && isfinite(x1) && isfinite(x2)) ? 0u : 1u;
-            esc = key - key_offsets[sc] == tab[sc].S.escape_key ? 1u : 0u;
+            const uint32_t q = __float_as_uint(sq) & 0x7FFFFFFFu;  // |v|^2 >= 0; a NaN keeps its payload above +inf
+            m = q > m ? q : m;
+            nb += (isfinite(a) && isfinite(b) && isfinite(c) && isfinite(x0) && isfinite(x1) && isfinite(x2)) ? 0u : 1u;
+            ne += keys[i] == escape ? 1u : 0u;
         }
-        // a wave of one scene reduces first; scene boundaries add per lane
-        const int s0 = __shfl(sc, 0, 64);
-        if (__ballot(act && sc != s0) == 0ull) {
-            uint32_t m = q, nb = bad, ne = esc;
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const uint32_t o = __shfl_xor(m, off, 64);
-                m = o > m ? o : m;
-                nb += __shfl_xor(nb, off, 64);
-                ne += __shfl_xor(ne, off, 64);
-            }
-            if (lane == 0) {
-                atomicMax(&out[3 * s0], m);
-                if (nb) atomicAdd(&out[3 * s0 + 1], nb);
-                if (ne) atomicAdd(&out[3 * s0 + 2], ne);
-            }
-        } else if (act) {
-            atomicMax(&out[3 * sc], q);
-            if (bad) atomicAdd(&out[3 * sc + 1], bad);
-            if (esc) atomicAdd(&out[3 * sc + 2], esc);
+        for (int off = 32; off > 0; off >>= 1) {
+            const uint32_t o = __shfl_xor(m, off, 64);
+            m = o > m ? o : m;
+            nb += __shfl_xor(nb, off, 64);
+            ne += __shfl_xor(ne, off, 64);
         }
+        if (lane == 0) {
+            part[wave][0] = m;
+            part[wave][1] = nb;
+            part[wave][2] = ne;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < 4; ++w) {
+                m = part[w][0] > m ? part[w][0] : m;
+                nb += part[w][1];
+                ne += part[w][2];
+            }
+            atomicMax(&out[3 * sc], m);
+            if (nb) atomicAdd(&out[3 * sc + 1], nb);
+            if (ne) atomicAdd(&out[3 * sc + 2], ne);
+        }
+        __syncthreads();
+        i0 = end;
     }
 }
 void launch_batch_health(const SceneEntry* tab, const uint32_t* key_offsets, int ns, int64_t ntot,
                          const uint32_t* keys, uint32_t* out, hipStream_t st) {
     if (ntot <= 0 || ns <= 0) return;
-    int64_t w = (ntot + 255) / 256;
-    if (w > 2048) w = 2048;
-    hipLaunchKernelGGL(k_batch_health, dim3((unsigned)w), dim3(256), 0, st, tab, key_offsets, ns, ntot, keys, out);
+    // about eight workgroups per compute unit, in whole rounds of 256 slots
+    const int64_t per = 256 * ((ntot + 256 * 2048 - 1) / (256 * 2048));
+    hipLaunchKernelGGL(k_batch_health, dim3((unsigned)((ntot + per - 1) / per)), dim3(256), 0, st, tab, key_offsets,
+                       ns, ntot, per, keys, out);
 }
 
 __global__ void k_debug_svd(const float* A, int64_t n, float* U, float* s, float* V) {
