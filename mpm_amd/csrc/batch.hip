@@ -131,6 +131,8 @@ struct Batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     Tune graph_tune;
+    bool graph_light = false;  // captured with the full sort in one launch
+    IncHistory updates;
     // stats and timing
     int64_t steps = 0;
     double last_step_ms = 0.0;
@@ -212,6 +214,12 @@ int ensure_capacity(Batch& b, int64_t n) {
     HIP_TRY(hipMemcpyAsync(b.moves_dev, &b.moves, sizeof(MoveList), hipMemcpyHostToDevice, b.st));
     HIP_TRY(hipMemsetAsync(b.plan, 0, kPlanWords * 4, b.st));  // no snapshot yet
     HIP_TRY(hipMemcpyAsync(b.plan + kPlanCap, &b.move_cap, 4, hipMemcpyHostToDevice, b.st));
+    if (!b.updates.host && (hipHostMalloc((void**)&b.updates.host, 64, hipHostMallocDefault) != hipSuccess ||
+                         hipEventCreateWithFlags(&b.updates.ev, hipEventDisableTiming) != hipSuccess))
+        (void)hipGetLastError();  // without the history the full sort stays one launch
+    b.updates.pending = false;
+    b.updates.prev_step = -1;  // the count begins anew
+    b.updates.mostly_updates = true;
     b.snap_ok = false;
     if ((rc = balloc(b, (void**)&b.items, (size_t)c * 8))) return rc;  // starts + blocks
     const int64_t hw = radix_hist_words(c);
@@ -443,8 +451,8 @@ int sync_members(Batch& b) {
 // fused: the fused transfer; scattered: every member's grid already holds
 // this step's P2G (else the step clears and scatters the others first);
 // full_sort: the step is known to sort in full (the snapshot was just
-// invalidated), else the radix launches use the light plan of a sort that
-// mostly returns at once.
+// invalidated), else the full sort is one launch that mostly returns at
+// once, while most steps update.
 // overlap: the grid clears run on the second stream (eager steps; a
 // captured step keeps them on the batch stream).
 void enqueue_step(Batch& b, bool fused, bool scattered, bool full_sort, bool overlap) {
@@ -468,7 +476,7 @@ void enqueue_step(Batch& b, bool fused, bool scattered, bool full_sort, bool ove
     uint32_t* const plan = b.incr ? b.plan : nullptr;
     if (plan) launch_inc_prepare(plan, b.moves, b.snap_k, b.snap_p, b.ntot, b.st);
     const int sel = radix_sort_pairs(b.kin, b.iota, b.ka, b.va, b.kb, b.vb, b.ntot, b.key_bits, b.hist, b.scan_temp,
-                                     b.st, ProfileHook{}, plan, plan && !full_sort);
+                                     b.st, ProfileHook{}, plan, plan && !full_sort && b.updates.mostly_updates);
     b.I.sorted_keys = sel ? b.kb : b.ka;
     b.I.perm = sel ? b.vb : b.va;
     if (plan) launch_inc_merge(plan, b.moves, b.snap_k, b.snap_p, b.ntot, sel ? b.kb : b.ka, sel ? b.vb : b.va, b.st);
@@ -586,6 +594,7 @@ int capture_step(Batch& b, bool fused) {
     if (e != hipSuccess) return fail(MPM_ERR_HIP, std::string("batch graph capture: ") + hipGetErrorString(e));
     HIP_TRY(hipGraphInstantiate(&b.gexec, b.graph, nullptr, nullptr, 0));
     b.graph_tune = b.tune;
+    b.graph_light = b.updates.mostly_updates;
     return MPM_OK;
 }
 
@@ -605,7 +614,9 @@ int run_steps(Batch& b, int n, bool graph) {
     auto t0 = std::chrono::steady_clock::now();
     for (int i = 0; i < n; ++i) {
         const bool first_scatter = fused && !scattered;
-        if (graph && !first_scatter && (!b.gexec || !(b.graph_tune == b.tune))) {
+        if (b.incr) sample_history(b.updates, b.plan, b.steps + i, b.st);
+        if (graph && !first_scatter &&
+            (!b.gexec || !(b.graph_tune == b.tune) || b.graph_light != b.updates.mostly_updates)) {
             if ((rc = capture_step(b, fused))) return rc;
         }
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -666,6 +677,8 @@ void batch_destroy(Batch* b) {
     }
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
+    if (b->updates.ev) (void)hipEventDestroy(b->updates.ev);
+    if (b->updates.host) (void)hipHostFree(b->updates.host);
     if (b->st) (void)hipStreamDestroy(b->st);
     delete b;
 }

@@ -363,25 +363,28 @@ void ensure_stress(Solver& s) {
 
 // Every 8 steps the count of incremental sorts is copied into pinned host
 // memory on the stream; once the copy has landed (an event query, no wait)
-// the share of updates since the previous reading sets few_passes: mostly
-// updates (>= 3/4) -> the full sort's kernels, which then mostly return at
-// once, use 3 passes instead of 4.  Only the speed depends on it.
-static void sample_inc_history(Solver& s) {
-    if (s.capturing || !s.inc_host || !s.inc_ev) return;
-    if (s.inc_pending && hipEventQuery(s.inc_ev) == hipSuccess) {
-        const uint32_t now = *reinterpret_cast<volatile uint32_t*>(s.inc_host);
-        if (s.inc_prev_step >= 0 && s.inc_copy_step > s.inc_prev_step)
-            s.few_passes = 4.0 * (double)(now - s.inc_prev) >= 3.0 * (double)(s.inc_copy_step - s.inc_prev_step);
-        s.inc_prev = now;
-        s.inc_prev_step = s.inc_copy_step;
-        s.inc_pending = false;
+// the share of updates since the previous reading sets mostly_updates: while
+// it is 3/4 or more (or not known yet), the full sort is one launch, which
+// mostly returns at once, else it is launched pass by pass.  Where it does run
+// the one launch takes the longer (1.1M keys: 250 us against 75; 8.4M: 800
+// against 310); where it does not, 5 us against 54 and more.  Only the speed
+// depends on it.
+void sample_history(IncHistory& h, const uint32_t* plan, int64_t steps, hipStream_t st) {
+    if (!h.host || !h.ev) return;
+    if (h.pending && hipEventQuery(h.ev) == hipSuccess) {
+        const uint32_t now = *reinterpret_cast<volatile uint32_t*>(h.host);
+        if (h.prev_step >= 0 && h.copy_step > h.prev_step)
+            h.mostly_updates = 4.0 * (double)(now - h.prev) >= 3.0 * (double)(h.copy_step - h.prev_step);
+        h.prev = now;
+        h.prev_step = h.copy_step;
+        h.pending = false;
     }
-    if (!s.inc_pending && s.steps - s.inc_copy_step >= 8) {
-        if (hipMemcpyAsync(s.inc_host, s.plan + kPlanIncSteps, 4, hipMemcpyDeviceToHost, s.st) != hipSuccess ||
-            hipEventRecord(s.inc_ev, s.st) != hipSuccess)
+    if (!h.pending && steps - h.copy_step >= 8) {
+        if (hipMemcpyAsync(h.host, plan + kPlanIncSteps, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+            hipEventRecord(h.ev, st) != hipSuccess)
             return;
-        s.inc_copy_step = s.steps;
-        s.inc_pending = true;
+        h.copy_step = steps;
+        h.pending = true;
     }
 }
 
@@ -401,17 +404,17 @@ static bool update_pays(const Solver& s) {
     return s.moves_seen < 0 || tiles * s.moves_seen <= kUpdateReads;
 }
 static void sample_moves(Solver& s) {
-    if (s.capturing || s.N < (int64_t(1) << 17) || !s.inc_host || !s.inc_ev) return;
-    if (s.inc_pending && hipEventQuery(s.inc_ev) == hipSuccess) {
-        s.moves_seen = *reinterpret_cast<volatile uint32_t*>(s.inc_host);
-        s.inc_pending = false;
+    if (s.capturing || s.N < (int64_t(1) << 17) || !s.updates.host || !s.updates.ev) return;
+    if (s.updates.pending && hipEventQuery(s.updates.ev) == hipSuccess) {
+        s.moves_seen = *reinterpret_cast<volatile uint32_t*>(s.updates.host);
+        s.updates.pending = false;
     }
-    if (!s.inc_pending && s.steps - s.inc_copy_step >= 8) {
-        if (hipMemcpyAsync(s.inc_host, s.plan + kPlanMoves, 4, hipMemcpyDeviceToHost, s.st) != hipSuccess ||
-            hipEventRecord(s.inc_ev, s.st) != hipSuccess)
+    if (!s.updates.pending && s.steps - s.updates.copy_step >= 8) {
+        if (hipMemcpyAsync(s.updates.host, s.plan + kPlanMoves, 4, hipMemcpyDeviceToHost, s.st) != hipSuccess ||
+            hipEventRecord(s.updates.ev, s.st) != hipSuccess)
             return;
-        s.inc_copy_step = s.steps;
-        s.inc_pending = true;
+        s.updates.copy_step = s.steps;
+        s.updates.pending = true;
     }
 }
 // The buffers of the update; without them (out of memory) every step sorts
@@ -435,8 +438,8 @@ static bool ensure_small_sort(Solver& s) {
     s.moves.pos = s.moves.slot + l;
     s.move_cap = small_list_cap(s.N);
     if (s.N >= (int64_t(1) << 17) &&
-        (hipHostMalloc((void**)&s.inc_host, 64, hipHostMallocDefault) != hipSuccess ||
-         hipEventCreateWithFlags(&s.inc_ev, hipEventDisableTiming) != hipSuccess))
+        (hipHostMalloc((void**)&s.updates.host, 64, hipHostMallocDefault) != hipSuccess ||
+         hipEventCreateWithFlags(&s.updates.ev, hipEventDisableTiming) != hipSuccess))
         (void)hipGetLastError();  // without the sample the update is taken every time
     launch_update_init(s.plan, s.moves_dev, s.moves, s.st);
     s.snap_ok = false;
@@ -498,7 +501,7 @@ static void seed_snapshot(Solver& s) {
 // at once.  Bit-identical to run_sort.
 void run_sort_incremental(Solver& s) {
     ProfileHook h = hook(s);
-    sample_inc_history(s);
+    if (!s.capturing) sample_history(s.updates, s.plan, s.steps, s.st);
     if (!s.keys_valid) {
         Scope sc(h, "keys");
         launch_keys(s.S, s.P, s.interp, s.kin, s.st);
@@ -511,7 +514,7 @@ void run_sort_incremental(Solver& s) {
         launch_inc_prepare(s.plan, s.moves, s.snap_k, s.snap_p, s.N, s.st);
     }
     const int sel = radix_sort_pairs(s.kin, s.iota, s.ka, s.va, s.kb, s.vb, s.N, s.key_bits, s.hist, s.scan_temp,
-                                     s.st, h, s.plan, s.few_passes);
+                                     s.st, h, s.plan, s.snap_ok && s.updates.mostly_updates);
     uint32_t* out_k = sel ? s.kb : s.ka;
     uint32_t* out_p = sel ? s.vb : s.va;
     s.I.sorted_keys = out_k;
@@ -775,8 +778,8 @@ int build(Solver& s, HostState& H, int run_init) {
         HIP_TRY(hipMemsetAsync(s.moves.ins, 0, tiles * kIncBucket * sizeof(uint2), s.st));
         if ((rc = dalloc(s, (void**)&s.moves_dev, sizeof(MoveList)))) return rc;
         HIP_TRY(hipMemcpyAsync(s.plan + kPlanCap, &s.move_cap, 4, hipMemcpyHostToDevice, s.st));
-        HIP_TRY(hipHostMalloc((void**)&s.inc_host, 64, hipHostMallocDefault));
-        HIP_TRY(hipEventCreateWithFlags(&s.inc_ev, hipEventDisableTiming));
+        HIP_TRY(hipHostMalloc((void**)&s.updates.host, 64, hipHostMallocDefault));
+        HIP_TRY(hipEventCreateWithFlags(&s.updates.ev, hipEventDisableTiming));
         HIP_TRY(hipMemcpyAsync(s.moves_dev, &s.moves, sizeof(MoveList), hipMemcpyHostToDevice, s.st));
         HIP_TRY(hipStreamSynchronize(s.st));  // the host copy is a member: it outlives the copy anyway
     }
@@ -833,8 +836,8 @@ void destroy(Solver* s) {
         (void)hipStreamDestroy(s->aux_st);
     }
     if (s->aux_fork) (void)hipEventDestroy(s->aux_fork);
-    if (s->inc_ev) (void)hipEventDestroy(s->inc_ev);
-    if (s->inc_host) (void)hipHostFree(s->inc_host);
+    if (s->updates.ev) (void)hipEventDestroy(s->updates.ev);
+    if (s->updates.host) (void)hipHostFree(s->updates.host);
     if (s->aux_join) (void)hipEventDestroy(s->aux_join);
     if (s->pos4_packed) (void)hipEventDestroy(s->pos4_packed);
     if (s->pos4_copied) (void)hipEventDestroy(s->pos4_copied);
@@ -1090,7 +1093,7 @@ MPM_API int mpm_step_graph(void* handle, int n) {
     // the captured step updates the last order, or sorts in full where that
     // is the shorter
     if (small && !s->snap_ok) seed_snapshot(*s);
-    if (!s->gexec) {
+    auto capture = [&]() -> int {
         const int prof = s->prof;  // no events inside the capture
         s->prof = 0;
         HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
@@ -1116,6 +1119,12 @@ MPM_API int mpm_step_graph(void* handle, int n) {
         s->graph_I = s->I;  // the sort buffers the replays write
         s->graph_grid = s->S.grid;
         s->graph_small = small;
+        s->graph_light = s->updates.mostly_updates;
+        return MPM_OK;
+    };
+    if (!s->gexec) {
+        const int rc = capture();
+        if (rc) return rc;
     }
     auto t0 = std::chrono::steady_clock::now();
     for (int i = 0; i < n; ++i) {
@@ -1126,6 +1135,14 @@ MPM_API int mpm_step_graph(void* handle, int n) {
             int rc = reorder_store(*s);
             if (rc) return rc;
             if (small) seed_snapshot(*s);
+        }
+        if (s->incr) {
+            sample_history(s->updates, s->plan, s->steps, s->st);
+            if (s->graph_light != s->updates.mostly_updates) {
+                drop_graph(*s);
+                const int rc = capture();
+                if (rc) return rc;
+            }
         }
         HIP_TRY(hipGraphLaunch(s->gexec, s->st));
         s->steps += 1;

@@ -129,6 +129,8 @@ enum PlanWord {
     kPlanCap = 3,       // capacity of one sub-list
     kPlanOverflow = 4,  // a sub-list or a snapshot tile's bucket overflowed
     kPlanMoves = 5,     // entries of the move list of the last sort
+    kPlanTicket = 8,    // the full sort in one launch: next piece of work,
+    kPlanDone = 32,     // pieces done per phase (zero between steps)
     kPlanLists = 64,    // the sub-list counters: word kPlanLists + r * kMoveCountStride
     kPlanWords = kPlanLists + kMoveLists * kMoveCountStride
 };

@@ -216,6 +216,7 @@ __global__ void __launch_bounds__(kScanWG) k_item_count(const uint32_t* __restri
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) moves += __shfl_xor(moves, off, 64);
             if (threadIdx.x == 0) plan[kPlanMoves] = moves;
+            if (threadIdx.x >= kPlanTicket && threadIdx.x < kPlanLists) plan[threadIdx.x] = 0u;  // the full sort's counters
         }
         if (threadIdx.x == 0) {
             plan[kPlanIncSteps] += plan_incremental(plan) ? 1u : 0u;

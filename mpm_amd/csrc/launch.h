@@ -24,13 +24,13 @@ int64_t scan_temp_words(int64_t n);
 // plan (device, may be null): every launch returns at once when the plan
 // words choose the incremental update (plan_incremental).
 void exclusive_scan(uint32_t* data, int64_t n, uint32_t* temp, uint32_t* total, hipStream_t st,
-                    const uint32_t* plan = nullptr, int max_wgs = 0);
+                    const uint32_t* plan = nullptr);
 int64_t radix_tiles(int64_t n);
 int64_t radix_hist_words(int64_t n);
-int radix_passes(int key_bits, int64_t n, bool few_passes = false);
+int radix_passes(int key_bits, int64_t n);
 int radix_sort_pairs(const uint32_t* kin, const uint32_t* vin, uint32_t* ka, uint32_t* va, uint32_t* kb, uint32_t* vb,
                      int64_t n, int key_bits, uint32_t* hist, uint32_t* scan_temp, hipStream_t st,
-                     const ProfileHook& prof, const uint32_t* plan = nullptr, bool few_passes = false);
+                     const ProfileHook& prof, uint32_t* plan = nullptr, bool one_launch = false);
 
 // ---- incsort.hip
 // plan words: reset the move counter and the overflow and set whether the

@@ -42,6 +42,18 @@ struct Pending {
     hipEvent_t a, b;
 };
 
+// How often the sort's update ran lately: every few steps the count of updates
+// is copied into pinned host memory (never waited for).
+struct IncHistory {
+    uint32_t* host = nullptr;
+    hipEvent_t ev = nullptr;
+    bool pending = false;
+    int64_t copy_step = 0, prev_step = -1;
+    uint32_t prev = 0;
+    bool mostly_updates = true;
+};
+void sample_history(IncHistory& h, const uint32_t* plan, int64_t steps, hipStream_t st);
+
 struct Solver {
     mpm_desc desc{};
     int interp = 0, apic = 0;
@@ -137,15 +149,7 @@ struct Solver {
     // length in a recent step, or -1
     bool small_sort = false;
     int64_t moves_seen = -1;
-    // how often the update ran lately: the incremental-sort count read back
-    // every few steps through pinned memory (never waited for); mostly
-    // updates -> the full sort's launches use fewer passes (few_passes)
-    uint32_t* inc_host = nullptr;
-    hipEvent_t inc_ev = nullptr;
-    bool inc_pending = false;
-    int64_t inc_copy_step = 0, inc_prev_step = -1;
-    uint32_t inc_prev = 0;
-    bool few_passes = false;
+    IncHistory updates;  // of a small scene: the buffers of its own sample
     // fused transfer (APIC folded step, linear or quadratic): G2P scatters
     // the next step's P2G into the second grid buffer (same size as the
     // first: the two alternate), which then becomes the grid.  prescat:
@@ -161,6 +165,7 @@ struct Solver {
     decltype(SceneDev::grid) grid2 = nullptr;
     decltype(SceneDev::touched) touched2 = nullptr;
     decltype(SceneDev::grid) graph_grid = nullptr;  // the grid buffer the captured step uses
+    bool graph_light = false;  // captured with the full sort in one launch
     bool graph_small = false;  // the captured step's sort is the small update
     // member of a batch that fuses its transfer: the batch table's grid of
     // this scene holds the P2G of its current particles (the table's grid
