@@ -37,6 +37,7 @@
 #include <stdint.h>
 
 #include "blockscan.h"
+#include "gridclear.h"
 #include "launch.h"
 
 namespace mpm {
@@ -353,20 +354,14 @@ __device__ __forceinline__ void update_inserted(const TileLds<TILE>& T, uint32_t
     }
 }
 
-// Clear of the touched blocks of a grid, 8 consecutive blocks per wave.
+// Clear of the touched blocks of a grid, one group of blocks per wave.
 __device__ __forceinline__ void clear_blocks(const GridClear& C, int64_t wave) {
     const int lane = threadIdx.x & 63;
-    const int64_t b0 = wave * 8;
-    uint64_t todo = __ballot(lane < 8 && b0 + lane < C.nsb && C.touched[b0 + lane] != 0u);
-    unsigned long long cnt = 0;
-    while (todo) {
-        const int64_t b = b0 + __builtin_ctzll(todo);
-        todo &= todo - 1;
-        const int64_t ni = b * 64 + lane;
-        cnt += (unsigned long long)__popcll(__ballot(C.grid[ni] > 0.0f));
-        for (int f = 0; f < C.nfields; ++f) C.grid[(int64_t)f * C.plane + ni] = 0.0f;
-        if (lane == 0) C.touched[b] = 0u;
-    }
+    const int64_t b0 = wave * kClearGroup;
+    const uint32_t todo = (uint32_t)__ballot(lane < kClearGroup && b0 + lane < C.nsb && C.touched[b0 + lane] != 0u);
+    if (!todo) return;
+    const unsigned long long cnt =
+        clear_group(C.grid, C.plane, C.touched, b0, todo, C.nfields, lane, C.active != nullptr);
     if (C.active && cnt && lane == 0) atomicAdd(C.active, cnt);
 }
 
@@ -519,7 +514,7 @@ void launch_sort_update(const uint32_t* plan, const MoveList& L, const uint32_t*
                         int64_t n, uint32_t* out_k, uint32_t* out_p, uint32_t* tmp_k, uint32_t* tmp_p,
                         const GridClear& clear, hipStream_t st) {
     const uint32_t tiles = (uint32_t)((n + kUpdateTile - 1) / kUpdateTile);
-    const int64_t waves = (clear.nsb + 7) / 8;
+    const int64_t waves = (clear.nsb + kClearGroup - 1) / kClearGroup;
     const uint32_t extra = (uint32_t)((waves + kIncWG / 64 - 1) / (kIncWG / 64));
     hipLaunchKernelGGL(k_sort_update, dim3(tiles + extra), dim3(kIncWG), 0, st, plan, L, snap_k, snap_p, (uint32_t)n,
                        tiles, out_k, out_p, tmp_k, tmp_p, clear);

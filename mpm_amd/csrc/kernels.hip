@@ -20,6 +20,7 @@
 
 #include "blockscan.h"
 #include "devmath.h"
+#include "gridclear.h"
 #include "launch.h"
 
 namespace mpm {
@@ -2259,51 +2260,23 @@ __device__ __forceinline__ void wg_count_add(unsigned long long* dst, unsigned l
     }
 }
 
-// Grid clear: one lane per storage block reads the touched flags
-// (coalesced); the wave then clears the touched blocks it found (64 nodes,
-// one per lane) and counts their nodes with mass > 0 (the active nodes of
-// the step that wrote them).  clear_block: one block (the batched clear).
-__device__ __forceinline__ unsigned long long clear_block(float* grid, int64_t plane, uint32_t* touched, int64_t b,
-                                                          int nfields, int lane) {
-    const int64_t ni = b * 64 + lane;
-    const unsigned long long c = (unsigned long long)__popcll(__ballot(grid[ni] > 0.0f));
-    for (int f = 0; f < nfields; ++f) grid[(int64_t)f * plane + ni] = 0.0f;
-    if (lane == 0) touched[b] = 0u;
-    return c;
-}
-
-// Each wave takes the touched blocks among 64 consecutive storage blocks,
-// kClearBatch at a time: their mass loads are all issued before the first
-// count waits on one, so a wave pays one memory latency per batch rather
-// than one per block.
-constexpr int kClearBatch = 8;
-__global__ void __launch_bounds__(256) k_clear(SceneDev S, int64_t nsb, int nfields, unsigned long long* active) {
+// Grid clear: a wave takes `groups` groups of kClearGroup consecutive storage
+// blocks, reads their flags together and clears the touched ones.  Latency
+// bounds it (flags, masses, stores, at most a few blocks each), so many waves
+// with little each: with 64 blocks per wave, one 256-byte store per plane and
+// block, the 2.1M slab's clear (160^3, 37 MB) took 41 us and the 8.4M slab's
+// (256^3, 100 MB, beside the sort) 50; 17 and 40 us now.
+__global__ void __launch_bounds__(256) k_clear(SceneDev S, int64_t nsb, int groups, int nfields,
+                                               unsigned long long* active) {
     const int lane = threadIdx.x & 63;
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint64_t todo = __ballot(b < nsb && S.touched[b] != 0u);
-    const int64_t wave0 = b - lane;
+    const int64_t b0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * groups * kClearGroup;
+    const int64_t b = b0 + lane;
+    uint64_t todo = __ballot(lane < groups * kClearGroup && b < nsb && S.touched[b] != 0u);
     unsigned long long cnt = 0;
-    while (todo) {
-        int64_t blk[kClearBatch];
-        float m[kClearBatch];
-#pragma unroll
-        for (int u = 0; u < kClearBatch; ++u) {
-            blk[u] = -1;
-            if (todo) {
-                blk[u] = wave0 + __builtin_ctzll(todo);
-                todo &= todo - 1;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kClearBatch; ++u) m[u] = blk[u] >= 0 ? S.grid[blk[u] * 64 + lane] : 0.0f;
-#pragma unroll
-        for (int u = 0; u < kClearBatch; ++u) {
-            if (blk[u] < 0) continue;
-            cnt += (unsigned long long)__popcll(__ballot(m[u] > 0.0f));
-            const int64_t ni = blk[u] * 64 + lane;
-            for (int f = 0; f < nfields; ++f) S.grid[(int64_t)f * S.plane + ni] = 0.0f;
-            if (lane == 0) S.touched[blk[u]] = 0u;
-        }
+    for (int64_t q = b0; todo; q += kClearGroup, todo >>= kClearGroup) {
+        const uint32_t mine = (uint32_t)todo & ((1u << kClearGroup) - 1u);
+        if (mine) cnt += clear_group((float*)S.grid, S.plane, (uint32_t*)S.touched, q, mine, nfields, lane,
+                                     active != nullptr);
     }
     if (active) wg_count_add(active, lane == 0 ? cnt : 0ull);
 }
@@ -2337,22 +2310,29 @@ __device__ __forceinline__ float MPM_GLOBAL* clear_grid_of(const SceneEntry& e, 
 __device__ __forceinline__ uint32_t MPM_GLOBAL* clear_touched_of(const SceneEntry& e, int mode) {
     return mode == 2 ? e.touched2 : e.S.touched;
 }
+// A wave takes kBatchClearGroups groups of blocks, as k_clear; a group of more
+// than one scene scene by scene.  Fewer blocks per wave repeat the search of
+// the scene (12.6M particles in 256 scenes, beside the sort: 216 us with 8
+// blocks per wave, 66 with 64; 97 with a search per lane and block by block).
+constexpr int kBatchClearGroups = 8;  // a block per lane: the scene is looked up once
+static_assert(kBatchClearGroups * kClearGroup == 64);
 __global__ void __launch_bounds__(256) k_clear_batch(const SceneEntry* __restrict__ tab,
                                                      const int64_t* __restrict__ block_start, int nscenes,
                                                      int nfields, int mode) {
     const int lane = threadIdx.x & 63;
-    const int64_t gb = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t gb0 = ((int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) *
+                        (kBatchClearGroups * kClearGroup);
+    const int64_t gb = gb0 + lane;
     const int64_t total = block_start[nscenes];
-    int sc = 0;
+    int sc = 0, hi = nscenes - 1;  // the first block's scene, by scalar loads
+    while (sc < hi) {
+        const int mid = (sc + hi + 1) >> 1;
+        if (block_start[mid] <= gb0) sc = mid;
+        else hi = mid - 1;
+    }
     bool t = false;
     if (gb < total) {
-        int lo = 0, hi = nscenes - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (block_start[mid] <= gb) lo = mid;
-            else hi = mid - 1;
-        }
-        sc = lo;
+        while (block_start[sc + 1] <= gb) ++sc;
         const bool take = mode != 1 || tab[sc].prescat == 0u;
         t = take && clear_touched_of(tab[sc], mode)[gb - block_start[sc]] != 0u;
     }
@@ -2365,17 +2345,18 @@ __global__ void __launch_bounds__(256) k_clear_batch(const SceneEntry* __restric
     unsigned long long run = 0;
     while (todo) {
         const int l = __builtin_ctzll(todo);
-        todo &= todo - 1;
         const int s = __builtin_amdgcn_readfirstlane(__shfl(sc, l, 64));
         if (s != cur) {
             if (lane == 0 && run) atomicAdd(tab[cur].active, run);
             cur = s;
             run = 0;
         }
-        const int64_t b = (gb - lane + l) - block_start[s];
-        const unsigned long long c = clear_block(clear_grid_of(tab[s], mode), tab[s].S.plane,
-                                                 clear_touched_of(tab[s], mode), b, nfields, lane);
-        if (mode != 2 || tab[s].prescat != 0u) run += c;
+        const int g = l & ~(kClearGroup - 1);  // the group's first lane
+        const uint64_t mine = todo & __ballot(sc == s) & (((1ull << kClearGroup) - 1ull) << g);
+        todo &= ~mine;
+        run += clear_group((float*)clear_grid_of(tab[s], mode), tab[s].S.plane,
+                           (uint32_t*)clear_touched_of(tab[s], mode), gb0 + g - block_start[s], (uint32_t)(mine >> g),
+                           nfields, lane, mode != 2 || tab[s].prescat != 0u);
     }
     if (lane == 0 && run) atomicAdd(tab[cur].active, run);
 }
@@ -2389,12 +2370,18 @@ static unsigned grid_pass_wgs(int64_t nsb) {
 
 void launch_clear(const SceneDev& S, int64_t nsb, int nfields, unsigned long long* active, hipStream_t st) {
     if (nsb <= 0) return;
-    hipLaunchKernelGGL(k_clear, dim3((unsigned)((nsb + 255) / 256)), dim3(256), 0, st, S, nsb, nfields, active);
+    // enough waves to fill the device, then two groups each
+    const int64_t g = nsb / ((int64_t)kClearGroup * 32 * device_cus());
+    const int groups = g < 1 ? 1 : (g > 2 ? 2 : (int)g);
+    const int64_t per = (int64_t)4 * groups * kClearGroup;  // blocks of a workgroup
+    hipLaunchKernelGGL(k_clear, dim3((unsigned)((nsb + per - 1) / per)), dim3(256), 0, st, S, nsb, groups, nfields,
+                       active);
 }
 void launch_clear_batch(const SceneEntry* tab, const int64_t* block_start, int nscenes, int64_t total_blocks,
                         int nfields, hipStream_t st, int mode) {
     if (total_blocks <= 0 || nscenes <= 0) return;
-    hipLaunchKernelGGL(k_clear_batch, dim3((unsigned)((total_blocks + 255) / 256)), dim3(256), 0, st, tab,
+    constexpr int64_t per = 4 * kBatchClearGroups * kClearGroup;
+    hipLaunchKernelGGL(k_clear_batch, dim3((unsigned)((total_blocks + per - 1) / per)), dim3(256), 0, st, tab,
                        block_start, nscenes, nfields, mode);
 }
 
