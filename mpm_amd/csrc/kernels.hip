@@ -1919,6 +1919,10 @@ __device__ __forceinline__ void scatter_moved(const SceneDev& S, float* grid, ui
 #ifndef MPM_G2P2G_WG
 #define MPM_G2P2G_WG 128
 #endif
+// Bound by VALU issue and the waits between (3 waves per SIMD).  The wait for
+// the staged words stands before the wave's stores, which count in the same
+// order (after them it waited for these too), and the wave's index is scalar,
+// so that its loop is: 8.4M particles 1205 -> 1169 us.
 // 3 waves per SIMD: the kernel needs ~162 VGPRs (at 128, 4 waves, ~24
 // spill); its LDS (19.6 KB per 128-thread workgroup) would allow 4.
 // BATCH: the items span the scenes of a batch; each item's scene, its
@@ -1938,7 +1942,7 @@ k_g2p2g(SceneDev S0, ParticlesDev P0, ItemsDev I, const SceneEntry* __restrict__
     __shared__ float stage[4 * TN];      // the next item's folded tile in flight
     __shared__ float pstage[PW * WG];    // Fe, Jp, mu0, lam0, V0 of each lane's particle
     __shared__ float otile[NW * 4 * TN];  // next step's sums, one tile per wave
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t nitems = *I.count;
     float* const ot = otile + wave * (4 * TN);
     ItemGeom gnext{};
@@ -2012,6 +2016,7 @@ k_g2p2g(SceneDev S0, ParticlesDev P0, ItemsDev I, const SceneEntry* __restrict__
                 __builtin_amdgcn_global_load_lds((const void*)(P.V0 + p), (lds_void*)(pst + 12 * 64), 4, 0, 0);
                 const float x0 = P.x[p], x1 = P.x[N + p], x2 = P.x[2 * N + p];
                 m = P.m[p];
+                const MaterialDev mat = P.mats[P.mat[p]];
                 float grad[3][3], Bm[3][3], v[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int r = 0; r < 3; ++r)
@@ -2032,6 +2037,9 @@ k_g2p2g(SceneDev S0, ParticlesDev P0, ItemsDev I, const SceneEntry* __restrict__
                     const float* const tq = tile + (((bz - g.oz) * T + (by - g.oy)) * T + (bx - g.ox));
                     apic_gather<W, T, TN>(tq, Nx, Ny, Nz, dNx, dNy, dNz, dxn, v, grad, Bm);
                 }
+                // the staged words and the material have landed by now; waited
+                // for after the stores below, the wave would wait for these too
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 store_m3(P.B, N, p, Bm);
                 if (pcollide) boundary_collision(S, x0 + S.dt * v[0], x1 + S.dt * v[1], x2 + S.dt * v[2], v[0], v[1], v[2]);
                 P.v[p] = v[0];
@@ -2046,12 +2054,9 @@ k_g2p2g(SceneDev S0, ParticlesDev P0, ItemsDev I, const SceneEntry* __restrict__
                 knew = koff + cell_key(S, xn[0], xn[1], xn[2], Stencil<INTERP>::SHIFT, Stencil<INTERP>::W);
                 next_keys[pbase + p] = knew;
                 // updateDeformationGradient and the stress of the new state
-                // (the material loaded before the wait below, and the move
-                // list's atomic issued after it: its result is used only
-                // after the F update)
-                const MaterialDev mat = P.mats[P.mat[p]];
+                // (the move list's atomic issued before: its result is used
+                // only after the F update)
                 float Fe[3][3];
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // staged words have landed
                 MoveTicket ticket{};
                 if (I.plan) ticket = move_begin(I, knew != kold);
                 float* const q = pst + lane;
