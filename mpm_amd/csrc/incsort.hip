@@ -32,7 +32,7 @@
 // and insertions were bucketed by counts, a scan in one workgroup and a second
 // pass (searches twice as long and two launches more).  Measured, the four
 // kernels before and the two now, us: 2.1M slab 38 -> 21, 8.4M slab 85 -> 45,
-// uneven batch of 12.6M 190 -> 90, served batch of 2.7M 114 -> 47.
+// uneven batch of 11.0M 190 -> 90, served batch of 2.6M 114 -> 47.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -72,7 +72,7 @@ __global__ void k_inc_set(uint32_t* plan, uint32_t snap_ok) {
 // bucket (its counter in a line of its own: atomics on one line wait for each
 // other).  The tiles' net change is counted apart, and only for the entries
 // that leave their tile, which about three in four do not: counted for all of
-// them in one word with the bucket's, a batch of 12.6M particles took 52 us
+// them in one word with the bucket's, a batch of 11.0M particles took 52 us
 // here, 31 now, the grid clear beside it.
 __global__ void __launch_bounds__(kIncWG) k_inc_route(uint32_t* __restrict__ plan, MoveList L,
                                                       const uint32_t* __restrict__ snap_k,

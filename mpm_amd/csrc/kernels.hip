@@ -273,7 +273,7 @@ __global__ void __launch_bounds__(kScanWG) k_item_emit(const uint32_t* __restric
     uint32_t k = first + block_exclusive_scan(c, ws, tot);
     if (RAW && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *item_count = first + tot;
     // the scene of the tile's first key, by scalar loads; the heads go on from
-    // there (12.6M keys of 256 scenes 23 us, 36 with a search per head)
+    // there (11.0M keys of 256 scenes 23 us, 36 with a search per head)
     int sc = 0;
     if (item_scene) {
         const uint32_t key = sk[(int64_t)blockIdx.x * kScanWG * IPT];
@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(kScanWG) k_item_emit(const uint32_t* __restric
 
 // Up to this many tiles the emit pass sums the tile counts before its own
 // itself (32 loads a thread at most), above it they are scanned first, two
-// launches more: 12.6M keys (3,077 tiles) 45 us with the scan, 36 without.
+// launches more: 11.0M keys (2,688 tiles) 45 us with the scan, 36 without.
 constexpr int64_t kEmitTiles = 8192;
 template <int IPT>
 static void launch_items_ipt(const uint32_t* sorted_keys, int64_t n, uint32_t* flags, uint32_t* scan_temp,
@@ -2334,7 +2334,7 @@ __device__ __forceinline__ uint32_t MPM_GLOBAL* clear_touched_of(const SceneEntr
 }
 // A wave takes kBatchClearGroups groups of blocks, as k_clear; a group of more
 // than one scene scene by scene.  Fewer blocks per wave repeat the search of
-// the scene (12.6M particles in 256 scenes, beside the sort: 216 us with 8
+// the scene (11.0M particles in 256 scenes, beside the sort: 216 us with 8
 // blocks per wave, 66 with 64; 97 with a search per lane and block by block).
 constexpr int kBatchClearGroups = 8;  // a block per lane: the scene is looked up once
 static_assert(kBatchClearGroups * kClearGroup == 64);
