@@ -271,9 +271,10 @@ __global__ void __launch_bounds__(kIncTile / kTileIPT) k_inc_merge(const uint32_
 // of the particles) and keeps what falls into its tile, instead of passes
 // that bucket the list first: the removals and insertions before the tile
 // give its offset, a scan over the tile's positions the place of every entry
-// in it.  Insertions at one place are put into scratch in arbitrary order,
-// then ranked among themselves.  The list holds every particle, so there is
-// no overflow and no full sort to launch beside it.
+// in it.  Up to kMatch insertions are ranked in LDS by counting; more (a layer
+// of a lattice that crosses cells in one step, a scene that loses its numbers
+// in one) are sorted in memory by the tile's workgroup.  The list holds every
+// particle, so there is no overflow and no full sort to launch beside it.
 // What bounds it: the list's entries times the tiles (12 bytes each, from
 // L2); the host takes the radix sort instead where that is the larger (see
 // run_sort_small).  Measured at 16,384 particles: six radix launches of 41 us
@@ -281,27 +282,32 @@ __global__ void __launch_bounds__(kIncTile / kTileIPT) k_inc_merge(const uint32_
 // A tile of the last order in LDS, the positions taken out of it and what is
 // put into it.
 constexpr int kMatch = 512;  // insertions kept in LDS
-template <int TILE>
 struct TileLds {
+    static constexpr int TILE = kUpdateTile;
     uint32_t sk[TILE], sp[TILE];
     uint32_t ins[TILE + 1];     // insertions at each place of the tile (TILE: after its last entry)
     uint32_t before[TILE + 1];  // removals (low 12 bits) and insertions before each place
     uint32_t gone[TILE / 32];   // removed positions
-    uint32_t mk[kMatch], ms[kMatch], place[kMatch];  // insertions and their places
-    uint32_t nmatch, ws[TILE / kTileIPT / 64];
-    // first place in the new order of what is inserted at place l; base: of the tile
+    union {
+        struct {
+            uint32_t mk[kMatch], ms[kMatch], place[kMatch];  // insertions and their places
+        };
+        struct {
+            uint32_t run[TILE / kTileIPT / 64][256], at[256];  // of sort_insertions
+        };
+    };
+    uint32_t nmatch, diff[2], ws[TILE / kTileIPT / 64];
+    // where the unmoved entry at place l goes in the new order, less the
+    // insertions at l; base: where the tile begins
     __device__ __forceinline__ uint32_t bucket(uint32_t base, uint32_t l) const {
         return base + l - (before[l] & 4095u) + (before[l] >> 12);
     }
 };
 
-// Counts the nm insertions in T.mk/T.ms into T.ins, scans the places and
-// writes the tile's unmoved entries; base: where the tile begins in the new
-// order.  Call it after a barrier; ends with T complete for every thread.
-template <int TILE>
-__device__ __forceinline__ void update_unmoved(TileLds<TILE>& T, uint32_t cnt, uint32_t nm, uint32_t n, uint32_t base,
-                                               uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_p) {
-    constexpr int IPT = kTileIPT, WG = TILE / IPT;
+// Counts the nm insertions in T.mk/T.ms into T.ins and scans the places.  Call
+// it after a barrier; ends with T complete for every thread.
+__device__ __forceinline__ void scan_places(TileLds& T, uint32_t cnt, uint32_t nm) {
+    constexpr int TILE = TileLds::TILE, IPT = kTileIPT, WG = TILE / IPT;
     static_assert(TILE <= 2048, "removals of a tile take 12 bits of `before`");
     const uint32_t tid = threadIdx.x;
     for (uint32_t q = tid; q < nm; q += WG) {
@@ -326,9 +332,13 @@ __device__ __forceinline__ void update_unmoved(TileLds<TILE>& T, uint32_t cnt, u
     for (int r = 0; r < IPT; ++r) T.before[tid * IPT + r] = (dpre + d[r]) | ((ipre + c[r]) << 12);
     if (tid == 0) T.before[TILE] = dsum | (isum << 12);
     __syncthreads();
+}
+// The tile's unmoved entries; base: where the tile begins in the new order.
+__device__ __forceinline__ void put_unmoved(const TileLds& T, uint32_t cnt, uint32_t n, uint32_t base,
+                                            uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_p) {
 #pragma unroll
-    for (int r = 0; r < IPT; ++r) {
-        const uint32_t i = tid + r * WG;
+    for (int r = 0; r < kTileIPT; ++r) {
+        const uint32_t i = threadIdx.x + r * (TileLds::TILE / kTileIPT);
         if (i >= cnt || ((T.gone[i >> 5] >> (i & 31u)) & 1u)) continue;
         const uint32_t dst = T.bucket(base, i) + T.ins[i];
         if (dst < n) {  // always, for a list that matches the snapshot
@@ -338,10 +348,9 @@ __device__ __forceinline__ void update_unmoved(TileLds<TILE>& T, uint32_t cnt, u
     }
 }
 // The nm insertions themselves, ranked among those at the same place.
-template <int TILE>
-__device__ __forceinline__ void update_inserted(const TileLds<TILE>& T, uint32_t nm, uint32_t n, uint32_t base,
-                                                uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_p) {
-    for (uint32_t q = threadIdx.x; q < nm; q += TILE / kTileIPT) {
+__device__ __forceinline__ void put_inserted(const TileLds& T, uint32_t nm, uint32_t n, uint32_t base,
+                                             uint32_t* __restrict__ out_k, uint32_t* __restrict__ out_p) {
+    for (uint32_t q = threadIdx.x; q < nm; q += TileLds::TILE / kTileIPT) {
         const uint32_t k = T.mk[q], s = T.ms[q], l = T.place[q];
         uint32_t rank = 0;
         if (T.ins[l] > 1u)
@@ -352,6 +361,98 @@ __device__ __forceinline__ void update_inserted(const TileLds<TILE>& T, uint32_t
             out_p[dst] = s;
         }
     }
+}
+
+// The m entries at (ak, ap) sorted by (key, slot) by one workgroup: a stable
+// pass per byte that is not the same in all of them, ping-pong with (bk, bp).
+// Returns whether the result is in (ak, ap).  Ends with a barrier.
+// Ranked by counting instead, every entry against all others at its place,
+// the time grew with the square (10,000 entries 58 ms, 40,000 0.93 s; now the
+// step that has them takes 0.22 and 0.68 ms): a layer of 4,096 particles made
+// its step of 60 us one of 14 ms.
+__device__ bool sort_insertions(TileLds& T, uint32_t* ak, uint32_t* ap, uint32_t* bk, uint32_t* bp, uint32_t m) {
+    constexpr uint32_t IPT = kTileIPT, WAVES = TileLds::TILE / kTileIPT / 64, CHUNK = TileLds::TILE;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    if (tid < 2u) T.diff[tid] = 0u;
+    __syncthreads();
+    const uint32_t k0 = ak[0], s0 = ap[0];
+    uint32_t dk = 0, ds = 0;
+    for (uint32_t q = tid; q < m; q += WAVES * 64u) {
+        dk |= ak[q] ^ k0;
+        ds |= ap[q] ^ s0;
+    }
+    if (dk) atomicOr(&T.diff[0], dk);
+    if (ds) atomicOr(&T.diff[1], ds);
+    __syncthreads();
+    dk = T.diff[0];
+    ds = T.diff[1];
+    bool in_a = true;
+    for (int byte = 0; byte < 8; ++byte) {  // of the slot, then of the key
+        const int shift = 8 * (byte & 3);
+        if ((((byte < 4 ? ds : dk) >> shift) & 255u) == 0u) continue;  // uniform
+        const uint32_t *ik = in_a ? ak : bk, *ip = in_a ? ap : bp;
+        uint32_t *ok = in_a ? bk : ak, *op = in_a ? bp : ap;
+        const uint32_t* const word = byte < 4 ? ip : ik;
+        // at: where each digit's next entry goes
+        static_assert(WAVES * 64u == 256u, "a thread per digit");
+        T.at[tid] = 0u;
+        __syncthreads();
+        for (uint32_t q = tid; q < m; q += 256u) atomicAdd(&T.at[(word[q] >> shift) & 255u], 1u);
+        __syncthreads();
+        uint32_t all;
+        const uint32_t first = block_exclusive_scan<256>(T.at[tid], T.ws, all);
+        T.at[tid] = first;
+        // a wave takes 4 x 64 consecutive entries of a chunk; run: its count
+        // of each digit so far, then where its first of the digit goes
+        for (uint32_t c0 = 0; c0 < m; c0 += CHUNK) {
+#pragma unroll
+            for (uint32_t w = 0; w < WAVES; ++w) T.run[w][tid] = 0u;
+            __syncthreads();
+            uint32_t k[IPT], s[IPT], d[IPT], rank[IPT];
+#pragma unroll
+            for (uint32_t r = 0; r < IPT; ++r) {
+                const uint32_t q = c0 + (wave * IPT + r) * 64u + lane, qc = q < m ? q : m - 1u;
+                k[r] = ik[qc];
+                s[r] = ip[qc];
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < IPT; ++r) {
+                const bool valid = c0 + (wave * IPT + r) * 64u + lane < m;
+                d[r] = ((byte < 4 ? s[r] : k[r]) >> shift) & 255u;
+                uint64_t same = __ballot(valid);
+#pragma unroll
+                for (int b = 0; b < 8; ++b) {
+                    const uint64_t set = __ballot((d[r] >> b) & 1u);
+                    same &= (d[r] >> b) & 1u ? set : ~set;
+                }
+                const uint32_t before = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+                rank[r] = before + (valid ? T.run[wave][d[r]] : 0u);
+                asm volatile("" ::: "memory");  // a wave's LDS accesses are in order
+                if (valid && before == 0u) T.run[wave][d[r]] += (uint32_t)__popcll(same);
+                asm volatile("" ::: "memory");
+            }
+            __syncthreads();
+            uint32_t to = T.at[tid];
+#pragma unroll
+            for (uint32_t w = 0; w < WAVES; ++w) {
+                const uint32_t c = T.run[w][tid];
+                T.run[w][tid] = to;
+                to += c;
+            }
+            T.at[tid] = to;
+            __syncthreads();
+#pragma unroll
+            for (uint32_t r = 0; r < IPT; ++r) {
+                if (c0 + (wave * IPT + r) * 64u + lane >= m) continue;
+                const uint32_t dst = T.run[wave][d[r]] + rank[r];
+                ok[dst] = k[r];
+                op[dst] = s[r];
+            }
+            __syncthreads();
+        }
+        in_a = !in_a;
+    }
+    return in_a;
 }
 
 // Clear of the touched blocks of a grid, one group of blocks per wave.
@@ -368,8 +469,8 @@ __device__ __forceinline__ void clear_blocks(const GridClear& C, int64_t wave) {
 __global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restrict__ plan, MoveList L,
                                                         const uint32_t* __restrict__ snap_k,
                                                         const uint32_t* __restrict__ snap_p, uint32_t n,
-                                                        uint32_t tiles, uint32_t* __restrict__ out_k,
-                                                        uint32_t* __restrict__ out_p, uint32_t* tmp_k,
+                                                        uint32_t tiles, uint32_t* out_k, uint32_t* out_p,
+                                                        uint32_t* tmp_k,
                                                         uint32_t* tmp_p, GridClear C) {
     if (blockIdx.x >= tiles) {
         clear_blocks(C, (int64_t)(blockIdx.x - tiles) * (kIncWG / 64) + (threadIdx.x >> 6));
@@ -377,7 +478,7 @@ __global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restri
     }
     constexpr int TILE = kUpdateTile, IPT = kTileIPT;
     static_assert(TILE == kIncWG * IPT);
-    __shared__ TileLds<TILE> T;
+    __shared__ TileLds T;
     uint32_t (&sk)[TILE] = T.sk, (&sp)[TILE] = T.sp, (&ins)[TILE + 1] = T.ins;
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
     const uint32_t i0 = t * TILE, cnt = n - i0 < TILE ? n - i0 : TILE;
@@ -461,44 +562,43 @@ __global__ void __launch_bounds__(kIncWG) k_sort_update(const uint32_t* __restri
     block_exclusive_scan(db, T.ws, dtot);
     block_exclusive_scan(ib, T.ws, itot);
     const uint32_t base = i0 - dtot + itot;
-    update_unmoved(T, cnt, nm < kMatch ? nm : kMatch, n, base, out_k, out_p);
+    scan_places(T, cnt, nm < kMatch ? nm : kMatch);
     if (nm <= (uint32_t)kMatch) {  // uniform
-        update_inserted(T, nm, n, base, out_k, out_p);
+        put_unmoved(T, cnt, n, base, out_k, out_p);
+        put_inserted(T, nm, n, base, out_k, out_p);
         return;
     }
-    // more: put into scratch in arbitrary order, then ranked.  Their places
-    // need sk again, which holds the cursors, so they are found in the
-    // snapshot in memory
+    // more: gathered in arbitrary order and sorted in the tile's part of the
+    // new order, in scratch and in the output (nothing else is there yet).
+    // The places ascend with the entries, so entry q goes to its place less
+    // the removals before it plus q.
+    if (base > n || nm > n - base) return;  // never, for a list that matches the snapshot
+    if (tid == 0) T.nmatch = 0u;
     __syncthreads();
-    uint32_t* const cur = sk;
-#pragma unroll
-    for (int r = 0; r < IPT; ++r) cur[tid + r * kIncWG] = 0u;
-    __shared__ uint32_t cur_last;
-    if (tid == 0) cur_last = 0u;
-    __syncthreads();
-    auto for_matches = [&](auto&& fn) {
-        for_list([&](uint32_t k, uint32_t s, uint32_t) {
-            if (side(k, s) == 0) fn(k, s, place_in_tile(snap_k + i0, snap_p + i0, cnt, k, s));
-        });
-    };
-    for_matches([&](uint32_t k, uint32_t s, uint32_t l) {
-        const uint32_t u = atomicAdd(l < TILE ? &cur[l] : &cur_last, 1u);
-        const uint32_t dst = T.bucket(base, l) + u;
-        if (dst >= n) return;
-        uint32_t* const ok = ins[l] == 1u ? out_k : tmp_k;
-        uint32_t* const op = ins[l] == 1u ? out_p : tmp_p;
-        ok[dst] = k;
-        op[dst] = s;
+    for_list([&](uint32_t k, uint32_t s, uint32_t) {
+        if (side(k, s) != 0) return;
+        const uint32_t q = base + atomicAdd(&T.nmatch, 1u);
+        tmp_k[q] = k;
+        tmp_p[q] = s;
     });
     __syncthreads();
-    for_matches([&](uint32_t k, uint32_t s, uint32_t l) {
-        const uint32_t c0 = ins[l], b0 = T.bucket(base, l);
-        if (c0 == 1u || b0 + c0 > n) return;
-        uint32_t rank = 0;
-        for (uint32_t u = 0; u < c0; ++u) rank += entry_less(tmp_k[b0 + u], tmp_p[b0 + u], k, s) ? 1u : 0u;
-        out_k[b0 + rank] = k;
-        out_p[b0 + rank] = s;
-    });
+    const bool in_tmp = sort_insertions(T, tmp_k + base, tmp_p + base, out_k + base, out_p + base, nm);
+    if (!in_tmp) {
+        for (uint32_t q = tid; q < nm; q += kIncWG) {
+            tmp_k[base + q] = out_k[base + q];
+            tmp_p[base + q] = out_p[base + q];
+        }
+        __syncthreads();
+    }
+    put_unmoved(T, cnt, n, base, out_k, out_p);
+    for (uint32_t q = tid; q < nm; q += kIncWG) {
+        const uint32_t k = tmp_k[base + q], s = tmp_p[base + q], l = place_in_tile(sk, sp, cnt, k, s);
+        const uint32_t dst = base + l - (T.before[l] & 4095u) + q;
+        if (dst < n) {
+            out_k[dst] = k;
+            out_p[dst] = s;
+        }
+    }
 }
 
 __global__ void k_update_init(uint32_t* plan, MoveList* dev, MoveList L) {
