@@ -132,6 +132,7 @@ struct Batch {
     hipGraphExec_t gexec = nullptr;
     Tune graph_tune;
     bool graph_light = false;  // captured with the full sort in one launch
+    ItemsDev graph_I{};        // the sort buffers the replays write
     IncHistory updates;
     // stats and timing
     int64_t steps = 0;
@@ -595,6 +596,7 @@ int capture_step(Batch& b, bool fused) {
     HIP_TRY(hipGraphInstantiate(&b.gexec, b.graph, nullptr, nullptr, 0));
     b.graph_tune = b.tune;
     b.graph_light = b.updates.mostly_updates;
+    b.graph_I = b.I;
     return MPM_OK;
 }
 
@@ -630,8 +632,12 @@ int run_steps(Batch& b, int n, bool graph) {
             launch_inc_set(b.plan, 0u, b.st);
             b.snap_ok = true;
         }
-        if (graph && !first_scatter) HIP_TRY(hipGraphLaunch(b.gexec, b.st));
-        else enqueue_step(b, fused, scattered, full_sort, true);
+        if (graph && !first_scatter) {
+            HIP_TRY(hipGraphLaunch(b.gexec, b.st));
+            b.I = b.graph_I;  // an eager step since the capture may have sorted into the other buffers
+        } else {
+            enqueue_step(b, fused, scattered, full_sort, true);
+        }
         if (e0 && e1) {
             HIP_TRY(hipEventRecord(e1, b.st));
             b.pending.push_back({e0, e1});
