@@ -171,7 +171,11 @@ void bfree(Batch& b, void*& p) {
 }
 
 void drop_graph(Batch& b) {
-    if (b.gexec) { (void)hipGraphExecDestroy(b.gexec); b.gexec = nullptr; }
+    if (b.gexec) {
+        (void)hipStreamSynchronize(b.st);  // replays of it may still be queued or running
+        (void)hipGraphExecDestroy(b.gexec);
+        b.gexec = nullptr;
+    }
     if (b.graph) { (void)hipGraphDestroy(b.graph); b.graph = nullptr; }
 }
 
@@ -411,8 +415,7 @@ int sync_members(Batch& b) {
             batch_unfuse_member(&b, s);  // fusion turned off (tune) or no longer possible
             if (s.grid2) {  // its second grid is not needed while a member (it returns on first use)
                 // the scene's own captured step may use either buffer: it is captured again
-                if (s.gexec) { (void)hipGraphExecDestroy(s.gexec); s.gexec = nullptr; }
-                if (s.graph) { (void)hipGraphDestroy(s.graph); s.graph = nullptr; }
+                drop_graph(s);
                 s.graph_grid = nullptr;
                 dfree(s, s.grid2);
                 dfree(s, s.touched2);

@@ -237,9 +237,15 @@ int dedupe_materials(Solver& s, int64_t n, const float* xi, const float* thc, co
 }
 
 // The captured step holds the particle descriptor (with the material table's
-// address) by value: a new table invalidates it.
-static void drop_graph(Solver& s) {
-    if (s.gexec) { (void)hipGraphExecDestroy(s.gexec); s.gexec = nullptr; }
+// address) by value: a new table invalidates it.  Replays of it may still be
+// queued or running (a call of step_graph does not wait for them, and captures
+// again between them): they end first.
+void drop_graph(Solver& s) {
+    if (s.gexec) {
+        (void)hipStreamSynchronize(s.st);
+        (void)hipGraphExecDestroy(s.gexec);
+        s.gexec = nullptr;
+    }
     if (s.graph) { (void)hipGraphDestroy(s.graph); s.graph = nullptr; }
 }
 
@@ -1200,8 +1206,7 @@ MPM_API int mpm_set_grid_record(void* handle, int enable) {
     if (s->record_grid == (enable != 0)) return MPM_OK;
     s->record_grid = enable != 0;
     // the captured step and a batch's launches depend on the mode
-    if (s->gexec) { (void)hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
-    if (s->graph) { (void)hipGraphDestroy(s->graph); s->graph = nullptr; }
+    drop_graph(*s);
     if (s->batch) batch_invalidate(s->batch);
     return MPM_OK;
 }
@@ -1279,8 +1284,7 @@ MPM_API int mpm_switch_particles_collision(void* handle) {
     GET_SOLVER(s, handle);
     s->S.particle_collision = s->S.particle_collision ? 0 : 1;
     s->desc.particle_collision = s->S.particle_collision;
-    if (s->gexec) { (void)hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
-    if (s->graph) { (void)hipGraphDestroy(s->graph); s->graph = nullptr; }
+    drop_graph(*s);
     return MPM_OK;
 }
 

@@ -193,6 +193,7 @@ struct Scope {
     ~Scope() { h.end(n); }
 };
 void run_clear(Solver& s);
+void drop_graph(Solver& s);  // waits for its replays
 void ensure_stress(Solver& s);
 void destroy(Solver* s);
 int finish(Solver& s);
