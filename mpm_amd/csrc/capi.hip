@@ -1141,6 +1141,9 @@ MPM_API int mpm_step_graph(void* handle, int n) {
             int rc = reorder_store(*s);
             if (rc) return rc;
             if (small) seed_snapshot(*s);
+            // the plan words say that the next replay sorts in full: a step
+            // captured now must not hold that too, or every replay would
+            else if (s->incr) s->snap_ok = true;
         }
         if (s->incr) {
             sample_history(s->updates, s->plan, s->steps, s->st);

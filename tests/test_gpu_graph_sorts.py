@@ -1,0 +1,49 @@
+"""The sort of a captured step over a long run: the form of it that most steps
+need is captured again in the middle of a call, and the updates go on
+afterwards.  How often the update ran is read back without waiting, so the
+calls below are short and waited for."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from mpm_amd import native as N
+from mpm_amd import scenes
+from mpm_amd.solver import Solver
+from oracle import pyoracle
+
+pytestmark = pytest.mark.gpu
+
+
+def replay(gpu, steps, per_call=4):
+    for _ in range(0, steps, per_call):
+        gpu.step_graph(per_call)
+        gpu.synchronize()
+    return gpu.stats()
+
+
+def check_order(gpu, desc, tag):
+    """One more replay: its order is the stable sort of the positions before it."""
+    pos = gpu.read_positions4()[:, :3]
+    gpu.step_graph(1)
+    keys, ids, seq = gpu.read_sort()
+    ref = pyoracle.keys(desc, pos[seq])
+    order = pyoracle.stable_argsort(ref)
+    assert np.array_equal(keys, ref[order]) and np.array_equal(ids, seq[order]), tag
+
+
+def test_capture_beside_a_reorder_keeps_the_update():
+    sc = scenes.apic_slab(seed=7, nx=128, ny=64, nz=128, res=128, dt=5e-5, sigma_v=2.0)
+    gpu = Solver(sc.desc, sc.particles)
+    # a reorder before every replay: each sorts in full, so the full sort is
+    # captured again pass by pass, in the same turn as a reorder
+    gpu.set_reorder_interval(1)
+    st = replay(gpu, 48)
+    assert st["incremental_sorts"] == 0 and st["graph_captures"] == 2
+    check_order(gpu, sc.desc, "full sorts")
+    # none any more: the replays update, and the light form comes back
+    gpu.set_reorder_interval(0)
+    st = replay(gpu, 48)
+    assert st["incremental_sorts"] >= 46 and st["graph_captures"] == 3, st
+    check_order(gpu, sc.desc, "updates")
+    gpu.close()
