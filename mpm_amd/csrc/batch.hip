@@ -30,6 +30,7 @@
 
 #include "devcache.h"
 #include "launch.h"
+#include "pinned.h"
 #include "solver_impl.h"
 
 namespace mpm {
@@ -133,7 +134,7 @@ struct Batch {
     Tune graph_tune;
     bool graph_light = false;  // captured with the full sort in one launch
     ItemsDev graph_I{};        // the sort buffers the replays write
-    IncHistory updates;
+    SortHistory history;
     // stats and timing
     int64_t steps = 0;
     double last_step_ms = 0.0;
@@ -219,12 +220,10 @@ int ensure_capacity(Batch& b, int64_t n) {
     HIP_TRY(hipMemcpyAsync(b.moves_dev, &b.moves, sizeof(MoveList), hipMemcpyHostToDevice, b.st));
     HIP_TRY(hipMemsetAsync(b.plan, 0, kPlanWords * 4, b.st));  // no snapshot yet
     HIP_TRY(hipMemcpyAsync(b.plan + kPlanCap, &b.move_cap, 4, hipMemcpyHostToDevice, b.st));
-    if (!b.updates.host && (hipHostMalloc((void**)&b.updates.host, 64, hipHostMallocDefault) != hipSuccess ||
-                         hipEventCreateWithFlags(&b.updates.ev, hipEventDisableTiming) != hipSuccess))
-        (void)hipGetLastError();  // without the history the full sort stays one launch
-    b.updates.pending = false;
-    b.updates.prev_step = -1;  // the count begins anew
-    b.updates.mostly_updates = true;
+    uint64_t* const word = b.history.word ? b.history.word : pinned::take();
+    if (word) *word = 0;  // the counts begin anew (the stream is synchronised above)
+    b.history = SortHistory{};
+    b.history.word = word;
     b.snap_ok = false;
     if ((rc = balloc(b, (void**)&b.items, (size_t)c * 8))) return rc;  // starts + blocks
     const int64_t hw = radix_hist_words(c);
@@ -480,7 +479,7 @@ void enqueue_step(Batch& b, bool fused, bool scattered, bool full_sort, bool ove
     uint32_t* const plan = b.incr ? b.plan : nullptr;
     if (plan) launch_inc_prepare(plan, b.moves, b.snap_k, b.snap_p, b.ntot, b.st);
     const int sel = radix_sort_pairs(b.kin, b.iota, b.ka, b.va, b.kb, b.vb, b.ntot, b.key_bits, b.hist, b.scan_temp,
-                                     b.st, ProfileHook{}, plan, plan && !full_sort && b.updates.mostly_updates);
+                                     b.st, ProfileHook{}, plan, plan && !full_sort && b.history.mostly_updates);
     b.I.sorted_keys = sel ? b.kb : b.ka;
     b.I.perm = sel ? b.vb : b.va;
     if (plan) launch_inc_merge(plan, b.moves, b.snap_k, b.snap_p, b.ntot, sel ? b.kb : b.ka, sel ? b.vb : b.va, b.st);
@@ -492,7 +491,7 @@ void enqueue_step(Batch& b, bool fused, bool scattered, bool full_sort, bool ove
         launch_reorder_chunk(b.tab, b.slot_scene, sel ? b.vb : b.va, b.chunk_bounds, b.chunk_rr, b.nchunks,
                              b.chunk_max, b.chunk_scratch, b.apic != 0, b.st);
     launch_items(b.I.sorted_keys, b.ntot, b.flags, b.scan_temp, b.items, b.counters, b.st, (uint32_t)b.tune.item_max,
-                 b.key_offsets, ns, b.item_scene, plan, plan ? b.moves.tnet : nullptr);
+                 b.key_offsets, ns, b.item_scene, plan, plan ? b.moves.tnet : nullptr, b.history.word);
     const SceneDev S0{};
     const ParticlesDev P0{};
     const int wgs = effective_wgs(b);
@@ -598,7 +597,7 @@ int capture_step(Batch& b, bool fused) {
     if (e != hipSuccess) return fail(MPM_ERR_HIP, std::string("batch graph capture: ") + hipGetErrorString(e));
     HIP_TRY(hipGraphInstantiate(&b.gexec, b.graph, nullptr, nullptr, 0));
     b.graph_tune = b.tune;
-    b.graph_light = b.updates.mostly_updates;
+    b.graph_light = b.history.mostly_updates;
     b.graph_I = b.I;
     return MPM_OK;
 }
@@ -619,9 +618,9 @@ int run_steps(Batch& b, int n, bool graph) {
     auto t0 = std::chrono::steady_clock::now();
     for (int i = 0; i < n; ++i) {
         const bool first_scatter = fused && !scattered;
-        if (b.incr) sample_history(b.updates, b.plan, b.steps + i, b.st);
+        if (b.incr) read_history(b.history);
         if (graph && !first_scatter &&
-            (!b.gexec || !(b.graph_tune == b.tune) || b.graph_light != b.updates.mostly_updates)) {
+            (!b.gexec || !(b.graph_tune == b.tune) || b.graph_light != b.history.mostly_updates)) {
             if ((rc = capture_step(b, fused))) return rc;
         }
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -679,6 +678,7 @@ void batch_destroy(Batch* b) {
     drop_graph(*b);
     for (auto& pr : b->pending) b->event_pool.push_back(pr.first), b->event_pool.push_back(pr.second);
     for (auto e : b->event_pool) (void)hipEventDestroy(e);
+    pinned::give(b->history.word);
     for (void* p : b->allocs) (void)devcache::release(p);  // the stream is synchronised above
     if (b->aux) {
         (void)hipStreamSynchronize(b->aux);
@@ -686,8 +686,6 @@ void batch_destroy(Batch* b) {
     }
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
-    if (b->updates.ev) (void)hipEventDestroy(b->updates.ev);
-    if (b->updates.host) (void)hipHostFree(b->updates.host);
     if (b->st) (void)hipStreamDestroy(b->st);
     delete b;
 }

@@ -23,6 +23,7 @@
 #include "devcache.h"
 #include "devmath.h"
 #include "launch.h"
+#include "pinned.h"
 #include "solver_impl.h"
 
 using namespace mpm;
@@ -367,38 +368,29 @@ void ensure_stress(Solver& s) {
     s.stress_valid = true;
 }
 
-// Every 8 steps the count of incremental sorts is copied into pinned host
-// memory on the stream; once the copy has landed (an event query, no wait)
-// the share of updates since the previous reading sets mostly_updates: while
+// Once the device has written a new word (every 8 sorts; no wait), the share
+// of updates since the one before sets mostly_updates: while
 // it is 3/4 or more (or not known yet), the full sort is one launch, which
 // mostly returns at once, else it is launched pass by pass.  Where it does run
 // the one launch takes the longer (1.1M keys: 250 us against 75; 8.4M: 800
 // against 310); where it does not, 5 us against 54 and more.  Only the speed
 // depends on it.
-void sample_history(IncHistory& h, const uint32_t* plan, int64_t steps, hipStream_t st) {
-    if (!h.host || !h.ev) return;
-    if (h.pending && hipEventQuery(h.ev) == hipSuccess) {
-        const uint32_t now = *reinterpret_cast<volatile uint32_t*>(h.host);
-        if (h.prev_step >= 0 && h.copy_step > h.prev_step)
-            h.mostly_updates = 4.0 * (double)(now - h.prev) >= 3.0 * (double)(h.copy_step - h.prev_step);
-        h.prev = now;
-        h.prev_step = h.copy_step;
-        h.pending = false;
-    }
-    if (!h.pending && steps - h.copy_step >= 8) {
-        if (hipMemcpyAsync(h.host, plan + kPlanIncSteps, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipEventRecord(h.ev, st) != hipSuccess)
-            return;
-        h.copy_step = steps;
-        h.pending = true;
-    }
+void read_history(SortHistory& h) {
+    if (!h.word) return;
+    const uint64_t w = __atomic_load_n(h.word, __ATOMIC_RELAXED);
+    const uint32_t sorts = (uint32_t)(w >> 32), updates = (uint32_t)w;
+    if (sorts == h.sorts) return;
+    if (h.sorts != 0u)
+        h.mostly_updates = 4.0 * (double)(updates - h.updates) >= 3.0 * (double)(sorts - h.sorts);
+    h.sorts = sorts;
+    h.updates = updates;
 }
 
 // The sort of a small scene's fused step: the update of the last order where
 // the snapshot is that order (the host knows), else the radix sort; both are
 // always right.  The update reads tiles x moves list entries, so above
 // kUpdateReads of them the radix sort is the shorter one: the list's length of
-// an earlier step decides, copied back every 8 steps without waiting.
+// an earlier step decides, which the device writes every 8 sorts.
 // Measured at 290,417 particles and 1% moves (284 tiles, 0.8M entry reads):
 // update 16 us with the grid's clear, radix 61 us in 12 launches; 8M reads are about 100 MB from L2.
 // Below 2^17 particles a list of every particle stays under the line.
@@ -410,18 +402,9 @@ static bool update_pays(const Solver& s) {
     return s.moves_seen < 0 || tiles * s.moves_seen <= kUpdateReads;
 }
 static void sample_moves(Solver& s) {
-    if (s.capturing || s.N < (int64_t(1) << 17) || !s.updates.host || !s.updates.ev) return;
-    if (s.updates.pending && hipEventQuery(s.updates.ev) == hipSuccess) {
-        s.moves_seen = *reinterpret_cast<volatile uint32_t*>(s.updates.host);
-        s.updates.pending = false;
-    }
-    if (!s.updates.pending && s.steps - s.updates.copy_step >= 8) {
-        if (hipMemcpyAsync(s.updates.host, s.plan + kPlanMoves, 4, hipMemcpyDeviceToHost, s.st) != hipSuccess ||
-            hipEventRecord(s.updates.ev, s.st) != hipSuccess)
-            return;
-        s.updates.copy_step = s.steps;
-        s.updates.pending = true;
-    }
+    if (!s.history.word) return;
+    const uint64_t w = __atomic_load_n(s.history.word, __ATOMIC_RELAXED);
+    if (w >> 32) s.moves_seen = (uint32_t)w;
 }
 // The buffers of the update; without them (out of memory) every step sorts
 // in full as before.
@@ -443,10 +426,7 @@ static bool ensure_small_sort(Solver& s) {
     s.moves.slot = s.moves.key + l;
     s.moves.pos = s.moves.slot + l;
     s.move_cap = small_list_cap(s.N);
-    if (s.N >= (int64_t(1) << 17) &&
-        (hipHostMalloc((void**)&s.updates.host, 64, hipHostMallocDefault) != hipSuccess ||
-         hipEventCreateWithFlags(&s.updates.ev, hipEventDisableTiming) != hipSuccess))
-        (void)hipGetLastError();  // without the sample the update is taken every time
+    if (s.N >= (int64_t(1) << 17)) s.history.word = pinned::take();  // without it the update is taken every time
     launch_update_init(s.plan, s.moves_dev, s.moves, s.st);
     s.snap_ok = false;
     s.small_sort = true;
@@ -454,7 +434,7 @@ static bool ensure_small_sort(Solver& s) {
 }
 static void run_sort_small(Solver& s, const GridClear& clear) {
     ProfileHook h = hook(s);
-    sample_moves(s);
+    if (!s.capturing) sample_moves(s);
     if (!s.keys_valid) {
         Scope sc(h, "keys");
         launch_keys(s.S, s.P, s.interp, s.kin, s.st);
@@ -487,7 +467,7 @@ static void run_sort_small(Solver& s, const GridClear& clear) {
     {
         Scope sc(h, "items");  // also empties the move list for this step's G2P
         launch_items(s.I.sorted_keys, s.N, s.flags, s.scan_temp, s.items, s.counters, s.st, 0, nullptr, 0, nullptr,
-                     s.plan);
+                     s.plan, nullptr, s.history.word);
     }
     s.sort_valid = true;
 }
@@ -507,7 +487,7 @@ static void seed_snapshot(Solver& s) {
 // at once.  Bit-identical to run_sort.
 void run_sort_incremental(Solver& s) {
     ProfileHook h = hook(s);
-    if (!s.capturing) sample_history(s.updates, s.plan, s.steps, s.st);
+    if (!s.capturing) read_history(s.history);
     if (!s.keys_valid) {
         Scope sc(h, "keys");
         launch_keys(s.S, s.P, s.interp, s.kin, s.st);
@@ -520,7 +500,7 @@ void run_sort_incremental(Solver& s) {
         launch_inc_prepare(s.plan, s.moves, s.snap_k, s.snap_p, s.N, s.st);
     }
     const int sel = radix_sort_pairs(s.kin, s.iota, s.ka, s.va, s.kb, s.vb, s.N, s.key_bits, s.hist, s.scan_temp,
-                                     s.st, h, s.plan, s.snap_ok && s.updates.mostly_updates);
+                                     s.st, h, s.plan, s.snap_ok && s.history.mostly_updates);
     uint32_t* out_k = sel ? s.kb : s.ka;
     uint32_t* out_p = sel ? s.vb : s.va;
     s.I.sorted_keys = out_k;
@@ -536,7 +516,7 @@ void run_sort_incremental(Solver& s) {
     {
         Scope sc(h, "items");  // also resets the plan words for this step's G2P
         launch_items(s.I.sorted_keys, s.N, s.flags, s.scan_temp, s.items, s.counters, s.st, 0, nullptr, 0, nullptr,
-                     s.plan, s.moves.tnet);
+                     s.plan, s.moves.tnet, s.history.word);
     }
     s.sort_valid = true;
 }
@@ -784,8 +764,7 @@ int build(Solver& s, HostState& H, int run_init) {
         HIP_TRY(hipMemsetAsync(s.moves.ins, 0, tiles * kIncBucket * sizeof(uint2), s.st));
         if ((rc = dalloc(s, (void**)&s.moves_dev, sizeof(MoveList)))) return rc;
         HIP_TRY(hipMemcpyAsync(s.plan + kPlanCap, &s.move_cap, 4, hipMemcpyHostToDevice, s.st));
-        HIP_TRY(hipHostMalloc((void**)&s.updates.host, 64, hipHostMallocDefault));
-        HIP_TRY(hipEventCreateWithFlags(&s.updates.ev, hipEventDisableTiming));
+        s.history.word = pinned::take();
         HIP_TRY(hipMemcpyAsync(s.moves_dev, &s.moves, sizeof(MoveList), hipMemcpyHostToDevice, s.st));
         HIP_TRY(hipStreamSynchronize(s.st));  // the host copy is a member: it outlives the copy anyway
     }
@@ -842,8 +821,6 @@ void destroy(Solver* s) {
         (void)hipStreamDestroy(s->aux_st);
     }
     if (s->aux_fork) (void)hipEventDestroy(s->aux_fork);
-    if (s->updates.ev) (void)hipEventDestroy(s->updates.ev);
-    if (s->updates.host) (void)hipHostFree(s->updates.host);
     if (s->aux_join) (void)hipEventDestroy(s->aux_join);
     if (s->pos4_packed) (void)hipEventDestroy(s->pos4_packed);
     if (s->pos4_copied) (void)hipEventDestroy(s->pos4_copied);
@@ -851,6 +828,7 @@ void destroy(Solver* s) {
     if (s->graph) (void)hipGraphDestroy(s->graph);
     for (auto& p : s->pending) s->event_pool.push_back(p.a), s->event_pool.push_back(p.b);
     for (auto e : s->event_pool) (void)hipEventDestroy(e);
+    pinned::give(s->history.word);
     for (void* p : s->allocs) (void)devcache::release(p);  // every stream of the scene is synchronised above
     if (s->st) (void)hipStreamDestroy(s->st);
     delete s;
@@ -923,6 +901,7 @@ MPM_API int mpm_get_cache_info(mpm_cache_info* out) {
 
 MPM_API int mpm_release_cache(void) {
     devcache::release_all();
+    pinned::release_all();
     return MPM_OK;
 }
 
@@ -1125,7 +1104,7 @@ MPM_API int mpm_step_graph(void* handle, int n) {
         s->graph_I = s->I;  // the sort buffers the replays write
         s->graph_grid = s->S.grid;
         s->graph_small = small;
-        s->graph_light = s->updates.mostly_updates;
+        s->graph_light = s->history.mostly_updates;
         return MPM_OK;
     };
     if (!s->gexec) {
@@ -1146,8 +1125,8 @@ MPM_API int mpm_step_graph(void* handle, int n) {
             else if (s->incr) s->snap_ok = true;
         }
         if (s->incr) {
-            sample_history(s->updates, s->plan, s->steps, s->st);
-            if (s->graph_light != s->updates.mostly_updates) {
+            read_history(s->history);
+            if (s->graph_light != s->history.mostly_updates) {
                 drop_graph(*s);
                 const int rc = capture();
                 if (rc) return rc;

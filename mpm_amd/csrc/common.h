@@ -120,6 +120,7 @@ constexpr int kMoveLists = 64;
 constexpr int kSmallLists = 16;   // of a scene below kIncMinParticles, each of small_list_cap(n) entries
 __host__ __device__ inline uint32_t small_list_cap(int64_t n) { return (uint32_t)((n + kSmallLists - 1) / kSmallLists); }
 constexpr int kMoveCountStride = 64;  // words between two sub-list counters
+constexpr uint32_t kHistorySorts = 8;  // sorts between two words for the host
 constexpr int kIncTile = 2048;    // snapshot entries per merge workgroup
 constexpr int kIncStage = 512;    // insertions that a tile's bucket holds
 constexpr int kIncBucket = kIncStage + 16;  // its size: a line for the fill count, then the entries
@@ -128,7 +129,7 @@ enum PlanWord {
     kPlanIncSteps = 2,  // steps sorted by the update since creation
     kPlanCap = 3,       // capacity of one sub-list
     kPlanOverflow = 4,  // a sub-list or a snapshot tile's bucket overflowed
-    kPlanMoves = 5,     // entries of the move list of the last sort
+    kPlanSorts = 5,     // steps sorted since creation
     kPlanTicket = 8,    // the full sort in one launch: next piece of work,
     kPlanDone = 32,     // pieces done per phase (zero between steps)
     kPlanLists = 64,    // the sub-list counters: word kPlanLists + r * kMoveCountStride

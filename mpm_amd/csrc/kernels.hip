@@ -202,25 +202,35 @@ __device__ __forceinline__ void item_heads(const uint32_t* __restrict__ sk, int6
 // first key).  plan (the incremental sort's words, or null): the sort of the
 // step is done, so the first workgroup counts an incremental sort and
 // resets the move counter for the step's G2P (and marks the snapshot that
-// the step's transfer takes as valid); the update's tile counts too.
+// the step's transfer takes as valid); the update's tile counts too.  history:
+// a word of host memory for every kHistorySorts-th sort (SortHistory); copied
+// from the plan words instead, it was a copy kernel of 4 us and a gap in the
+// stream of 6 to 11 every eighth step.
 template <int IPT>
 __global__ void __launch_bounds__(kScanWG) k_item_count(const uint32_t* __restrict__ sk, int64_t n,
                                                         uint32_t item_max, uint32_t* __restrict__ partial,
                                                         uint32_t* __restrict__ plan,
-                                                        uint32_t* __restrict__ tile_net, uint32_t inc_tiles) {
+                                                        uint32_t* __restrict__ tile_net, uint32_t inc_tiles,
+                                                        uint64_t* __restrict__ history) {
     __shared__ uint32_t ws[kScanWG / 64];
     for (uint32_t t = blockIdx.x * kScanWG + threadIdx.x; t < inc_tiles; t += gridDim.x * kScanWG) tile_net[t] = 0u;
     if (plan && blockIdx.x == 0) {
+        uint32_t moves = 0;
         if (threadIdx.x < kMoveLists) {  // one wave
-            uint32_t moves = plan[kPlanLists + threadIdx.x * kMoveCountStride];
+            moves = plan[kPlanLists + threadIdx.x * kMoveCountStride];
             plan[kPlanLists + threadIdx.x * kMoveCountStride] = 0u;
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) moves += __shfl_xor(moves, off, 64);
-            if (threadIdx.x == 0) plan[kPlanMoves] = moves;
             if (threadIdx.x >= kPlanTicket && threadIdx.x < kPlanLists) plan[threadIdx.x] = 0u;  // the full sort's counters
         }
         if (threadIdx.x == 0) {
-            plan[kPlanIncSteps] += plan_incremental(plan) ? 1u : 0u;
+            const uint32_t sorts = plan[kPlanSorts] + 1u;
+            const uint32_t updates = plan[kPlanIncSteps] + (plan_incremental(plan) ? 1u : 0u);
+            plan[kPlanSorts] = sorts;
+            plan[kPlanIncSteps] = updates;
+            if (history && sorts % kHistorySorts == 0u)
+                __hip_atomic_store(history, (uint64_t)sorts << 32 | (tile_net ? updates : moves), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_SYSTEM);
             plan[kPlanSnapOk] = 1u;
             plan[kPlanOverflow] = 0u;
         }
@@ -309,12 +319,12 @@ template <int IPT>
 static void launch_items_ipt(const uint32_t* sorted_keys, int64_t n, uint32_t* flags, uint32_t* scan_temp,
                              uint32_t* items, uint32_t* item_count, hipStream_t st, uint32_t item_max,
                              const uint32_t* key_offsets, int nscenes, uint32_t* item_scene, uint32_t* plan,
-                             uint32_t* tile_net) {
+                             uint32_t* tile_net, uint64_t* history) {
     const int64_t tiles = (n + kScanWG * IPT - 1) / (kScanWG * IPT);
     // flags[0..tiles) holds the tile head counts (then, for many tiles,
     // their exclusive scan)
     hipLaunchKernelGGL(k_item_count<IPT>, dim3((unsigned)tiles), dim3(kScanWG), 0, st, sorted_keys, n, item_max,
-                       flags, plan, tile_net, tile_net ? inc_tiles(n) : 0u);
+                       flags, plan, tile_net, tile_net ? inc_tiles(n) : 0u, history);
     if (tiles <= kEmitTiles) {
         hipLaunchKernelGGL((k_item_emit<true, IPT>), dim3((unsigned)tiles), dim3(kScanWG), 0, st, sorted_keys, n,
                            item_max, flags, items, key_offsets, nscenes, item_scene, item_count);
@@ -327,7 +337,7 @@ static void launch_items_ipt(const uint32_t* sorted_keys, int64_t n, uint32_t* f
 
 void launch_items(const uint32_t* sorted_keys, int64_t n, uint32_t* flags, uint32_t* scan_temp, uint32_t* items,
                   uint32_t* item_count, hipStream_t st, uint32_t item_max, const uint32_t* key_offsets,
-                  int nscenes, uint32_t* item_scene, uint32_t* plan, uint32_t* tile_net) {
+                  int nscenes, uint32_t* item_scene, uint32_t* plan, uint32_t* tile_net, uint64_t* history) {
     if (n <= 0) return;
     if (item_max == 0) {
         // a multiple of 64 up to kItemMax that still gives about four items
@@ -339,10 +349,10 @@ void launch_items(const uint32_t* sorted_keys, int64_t n, uint32_t* flags, uint3
     // 4 keys per thread up to 2M keys, then 16
     if (n <= (int64_t)2048 * kScanWG * 4)
         launch_items_ipt<4>(sorted_keys, n, flags, scan_temp, items, item_count, st, item_max, key_offsets, nscenes,
-                            item_scene, plan, tile_net);
+                            item_scene, plan, tile_net, history);
     else
         launch_items_ipt<16>(sorted_keys, n, flags, scan_temp, items, item_count, st, item_max, key_offsets, nscenes,
-                             item_scene, plan, tile_net);
+                             item_scene, plan, tile_net, history);
 }
 
 // ------------------------------------------------------- item decoding

@@ -84,11 +84,12 @@ void launch_iota(uint32_t* p, int64_t n, hipStream_t st);
 // unit for small n).  For a batch, key_offsets[nscenes] (ascending) gives
 // each item's scene in item_scene.  plan: the incremental sort's words, reset
 // for the step's G2P, with the tiles' net counts, zeroed (null: a small
-// scene's update has none).
+// scene's update has none).  history (with plan): the host's word on the sorts
+// (SortHistory), or null.
 void launch_items(const uint32_t* sorted_keys, int64_t n, uint32_t* flags, uint32_t* scan_temp, uint32_t* items,
                   uint32_t* item_count, hipStream_t st, uint32_t item_max = 0, const uint32_t* key_offsets = nullptr,
                   int nscenes = 0, uint32_t* item_scene = nullptr, uint32_t* plan = nullptr,
-                  uint32_t* tile_net = nullptr);
+                  uint32_t* tile_net = nullptr, uint64_t* history = nullptr);
 
 // grid_wgs: persistent workgroups; 0 = one resident round (occupancy of the
 // kernel instance x compute units).

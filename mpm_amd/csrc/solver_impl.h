@@ -42,17 +42,16 @@ struct Pending {
     hipEvent_t a, b;
 };
 
-// How often the sort's update ran lately: every few steps the count of updates
-// is copied into pinned host memory (never waited for).
-struct IncHistory {
-    uint32_t* host = nullptr;
-    hipEvent_t ev = nullptr;
-    bool pending = false;
-    int64_t copy_step = 0, prev_step = -1;
-    uint32_t prev = 0;
+// How the planned sorts went lately: a pinned word (pinned.h) that the item
+// count of every kHistorySorts-th sort writes (sorts << 32 | updates so far;
+// of a small scene: | moves of that sort) and the host reads without a wait.
+// Without a word (null) the choices below stay as they begin.
+struct SortHistory {
+    uint64_t* word = nullptr;
+    uint32_t sorts = 0, updates = 0;  // as read last
     bool mostly_updates = true;
 };
-void sample_history(IncHistory& h, const uint32_t* plan, int64_t steps, hipStream_t st);
+void read_history(SortHistory& h);
 
 struct Solver {
     mpm_desc desc{};
@@ -149,7 +148,7 @@ struct Solver {
     // length in a recent step, or -1
     bool small_sort = false;
     int64_t moves_seen = -1;
-    IncHistory updates;  // of a small scene: the buffers of its own sample
+    SortHistory history;
     // fused transfer (APIC folded step, linear or quadratic): G2P scatters
     // the next step's P2G into the second grid buffer (same size as the
     // first: the two alternate), which then becomes the grid.  prescat:

@@ -11,6 +11,7 @@ from mpm_amd import native as N
 from mpm_amd import scenes
 from mpm_amd.solver import Solver
 from oracle import pyoracle
+from tests.test_gpu_batch_replay import check_step, make_batch
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +48,27 @@ def test_capture_beside_a_reorder_keeps_the_update():
     assert st["incremental_sorts"] >= 46 and st["graph_captures"] == 3, st
     check_order(gpu, sc.desc, "updates")
     gpu.close()
+
+
+def test_batch_between_full_sorts_and_updates():
+    # 0.4 cells per step: tiles of the order draw more than their buckets hold,
+    # every replay sorts in full (captured again pass by pass); then at rest
+    b, scs, solvers, seqs = make_batch((3000, 2500, 4000), velocity=(0.4e4 / 32, 0.0, -0.1e4 / 32))
+
+    def run(steps):
+        for _ in range(0, steps, 4):
+            b.step_graph(4)
+            b.synchronize()
+        check_step(b, scs, solvers, seqs, lambda: b.step_graph(1), "replay")
+        check_step(b, scs, solvers, seqs, lambda: b.step(1), "eager")
+        return b.info()["incremental_sorts"]
+
+    assert run(20) == 0
+    for s in solvers:
+        st = s.read_particles()
+        st.velocity[:] = 0.0
+        s.write_particles(st)
+    assert run(40) >= 38
+    b.close()
+    for s in solvers:
+        s.close()
