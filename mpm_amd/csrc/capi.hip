@@ -390,21 +390,20 @@ void read_history(SortHistory& h) {
 // the snapshot is that order (the host knows), else the radix sort; both are
 // always right.  The update reads tiles x moves list entries, so above
 // kUpdateReads of them the radix sort is the shorter one: the list's length of
-// an earlier step decides, which the device writes every 8 sorts.
+// an earlier step decides, which the device writes every 8 sorts; back at half
+// of them, so that a captured step is not captured again and again.
 // Measured at 290,417 particles and 1% moves (284 tiles, 0.8M entry reads):
 // update 16 us with the grid's clear, radix 61 us in 12 launches; 8M reads are about 100 MB from L2.
 // Below 2^17 particles a list of every particle stays under the line.
 // clear: a grid to clear in the same launch (cleared by its own where the
 // radix sort runs).
 constexpr int64_t kUpdateReads = int64_t(1) << 23;
-static bool update_pays(const Solver& s) {
-    const int64_t tiles = (s.N + kUpdateTile - 1) / kUpdateTile;
-    return s.moves_seen < 0 || tiles * s.moves_seen <= kUpdateReads;
-}
 static void sample_moves(Solver& s) {
     if (!s.history.word) return;
     const uint64_t w = __atomic_load_n(s.history.word, __ATOMIC_RELAXED);
-    if (w >> 32) s.moves_seen = (uint32_t)w;
+    if ((w >> 32) == 0) return;
+    const int64_t reads = (s.N + kUpdateTile - 1) / kUpdateTile * (int64_t)(uint32_t)w;
+    s.update_pays = reads <= (s.update_pays ? kUpdateReads : kUpdateReads / 2);
 }
 // The buffers of the update; without them (out of memory) every step sorts
 // in full as before.
@@ -442,7 +441,7 @@ static void run_sort_small(Solver& s, const GridClear& clear) {
         s.snap_ok = false;
     }
     // (profile level 1 times the launch groups apart: clear and full sort)
-    if (s.snap_ok && s.prof != 1 && update_pays(s)) {
+    if (s.snap_ok && s.prof != 1 && s.update_pays) {
         Scope sc(h, "sort_incr");
         launch_sort_update(s.plan, s.moves, s.snap_k, s.snap_p, s.N, s.ka, s.va, s.kb, s.vb, clear, s.st);
         s.I.sorted_keys = s.ka;
@@ -1076,7 +1075,7 @@ MPM_API int mpm_step_graph(void* handle, int n) {
     const bool small = ensure_small_sort(*s);
     if (s->gexec && small != s->graph_small) drop_graph(*s);  // captured before the update had its buffers
     // the captured step updates the last order, or sorts in full where that
-    // is the shorter
+    // is the shorter (captured again when that changes)
     if (small && !s->snap_ok) seed_snapshot(*s);
     auto capture = [&]() -> int {
         const int prof = s->prof;  // no events inside the capture
@@ -1105,6 +1104,7 @@ MPM_API int mpm_step_graph(void* handle, int n) {
         s->graph_grid = s->S.grid;
         s->graph_small = small;
         s->graph_light = s->history.mostly_updates;
+        s->graph_update = s->update_pays;
         return MPM_OK;
     };
     if (!s->gexec) {
@@ -1124,13 +1124,12 @@ MPM_API int mpm_step_graph(void* handle, int n) {
             // captured now must not hold that too, or every replay would
             else if (s->incr) s->snap_ok = true;
         }
-        if (s->incr) {
-            read_history(s->history);
-            if (s->graph_light != s->history.mostly_updates) {
-                drop_graph(*s);
-                const int rc = capture();
-                if (rc) return rc;
-            }
+        if (s->incr) read_history(s->history);
+        else if (small) sample_moves(*s);
+        if (s->graph_light != s->history.mostly_updates || s->graph_update != s->update_pays) {
+            drop_graph(*s);
+            const int rc = capture();
+            if (rc) return rc;
         }
         HIP_TRY(hipGraphLaunch(s->gexec, s->st));
         s->steps += 1;

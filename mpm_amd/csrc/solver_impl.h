@@ -144,10 +144,10 @@ struct Solver {
     uint32_t move_cap = 0;          // capacity of one sub-list (also in the plan words)
     // a scene below kIncMinParticles: the update in one launch
     // (launch_sort_update) on the same snapshot, plan words and list (its own
-    // sub-lists; allocated at the first fused step); moves_seen: the list's
-    // length in a recent step, or -1
+    // sub-lists; allocated at the first fused step); update_pays: shorter than
+    // the radix sort, by the list's length in a recent step
     bool small_sort = false;
-    int64_t moves_seen = -1;
+    bool update_pays = true;
     SortHistory history;
     // fused transfer (APIC folded step, linear or quadratic): G2P scatters
     // the next step's P2G into the second grid buffer (same size as the
@@ -165,7 +165,8 @@ struct Solver {
     decltype(SceneDev::touched) touched2 = nullptr;
     decltype(SceneDev::grid) graph_grid = nullptr;  // the grid buffer the captured step uses
     bool graph_light = false;  // captured with the full sort in one launch
-    bool graph_small = false;  // the captured step's sort is the small update
+    bool graph_small = false;  // captured with the small update's buffers
+    bool graph_update = true;  // captured while update_pays
     // member of a batch that fuses its transfer: the batch table's grid of
     // this scene holds the P2G of its current particles (the table's grid
     // and grid2 may be swapped relative to S.grid / grid2 here, by the

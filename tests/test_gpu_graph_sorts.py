@@ -72,3 +72,33 @@ def test_batch_between_full_sorts_and_updates():
     b.close()
     for s in solvers:
         s.close()
+
+
+@pytest.mark.parametrize("graph", [True, False], ids=["graph", "eager"])
+def test_small_scene_between_radix_sort_and_update(graph):
+    # 2^23 entry reads are the line: 196 tiles x 40% of 200k particles are
+    # twice that, a scene at rest reads nothing
+    sc = scenes.snow_cube(seed=9, n=200_000, res=64, lo=0.25, hi=0.5, transfer=N.PIC_FLIP, dt=1e-4,
+                          velocity=(0.4e4 / 64, 0.0, 0.0))
+    gpu = Solver(sc.desc, sc.particles)
+    step = gpu.step_graph if graph else gpu.step
+
+    def run(steps):
+        for _ in range(0, steps, 4):
+            step(4)
+            gpu.synchronize()
+        for k in range(2):
+            pos = gpu.read_positions4()[:, :3]
+            step(1)
+            keys, ids, seq = gpu.read_sort()
+            ref = pyoracle.keys(sc.desc, pos[seq])
+            order = pyoracle.stable_argsort(ref)
+            assert np.array_equal(keys, ref[order]) and np.array_equal(ids, seq[order]), k
+        return gpu.stats()["graph_captures"]
+
+    assert run(20) == (2 if graph else 0)
+    st = gpu.read_particles()
+    st.velocity[:] = 0.0
+    gpu.write_particles(st)
+    assert run(24) == (3 if graph else 0)
+    gpu.close()
