@@ -388,22 +388,29 @@ void read_history(SortHistory& h) {
 
 // The sort of a small scene's fused step: the update of the last order where
 // the snapshot is that order (the host knows), else the radix sort; both are
-// always right.  The update reads tiles x moves list entries, so above
-// kUpdateReads of them the radix sort is the shorter one: the list's length of
-// an earlier step decides, which the device writes every 8 sorts; back at half
-// of them, so that a captured step is not captured again and again.
-// Measured at 290,417 particles and 1% moves (284 tiles, 0.8M entry reads):
-// update 16 us with the grid's clear, radix 61 us in 12 launches; 8M reads are about 100 MB from L2.
-// Below 2^17 particles a list of every particle stays under the line.
+// always right.  Every workgroup of the update reads the whole list and ranks
+// what falls into its tile, so with many moves the radix sort is the shorter
+// one: the list's length of an earlier step decides, which the device writes
+// every 8 sorts; back at half the line, so that a captured step is not
+// captured again and again.
+// Measured, a whole step with the update against one with the radix sort, by
+// the share of particles that change cell, us (PIC-FLIP):
+//   16,384: 10% 51 / 75, 20% 61 / 75, 25% 82 / 75, 50% 117 / 75
+//   70,000: 15% 77 / 99, 20% 86 / 99, 25% 109 / 100 (100,000: 20% 102 / 105)
+//   200,000: 10% 110 / 130, 20% 153 / 130; 400,000: 5% 150 / 173, 10% 178 / 174
+//   1,000,000: 1% 199 / 247, 5% 253 / 252, 10% 314 / 253
+// Up to about 100,000 the ranking in the tiles takes over at a fifth of the
+// particles (1,000 to 16,384 the same; 500: a half), above it the reads, about 1.6 us per
+// 1,000 moves, at what the radix sort costs more.
 // clear: a grid to clear in the same launch (cleared by its own where the
 // radix sort runs).
-constexpr int64_t kUpdateReads = int64_t(1) << 23;
+static int64_t update_moves(int64_t n) { return std::max<int64_t>(250, std::min(n / 5, 20000 + n / 32)); }
 static void sample_moves(Solver& s) {
     if (!s.history.word) return;
     const uint64_t w = __atomic_load_n(s.history.word, __ATOMIC_RELAXED);
     if ((w >> 32) == 0) return;
-    const int64_t reads = (s.N + kUpdateTile - 1) / kUpdateTile * (int64_t)(uint32_t)w;
-    s.update_pays = reads <= (s.update_pays ? kUpdateReads : kUpdateReads / 2);
+    const int64_t line = update_moves(s.N);
+    s.update_pays = (int64_t)(uint32_t)w <= (s.update_pays ? line : line / 2);
 }
 // The buffers of the update; without them (out of memory) every step sorts
 // in full as before.
@@ -425,7 +432,7 @@ static bool ensure_small_sort(Solver& s) {
     s.moves.slot = s.moves.key + l;
     s.moves.pos = s.moves.slot + l;
     s.move_cap = small_list_cap(s.N);
-    if (s.N >= (int64_t(1) << 17)) s.history.word = pinned::take();  // without it the update is taken every time
+    s.history.word = pinned::take();  // without it the update is taken every time
     launch_update_init(s.plan, s.moves_dev, s.moves, s.st);
     s.snap_ok = false;
     s.small_sort = true;

@@ -275,9 +275,9 @@ __global__ void __launch_bounds__(kIncTile / kTileIPT) k_inc_merge(const uint32_
 // of a lattice that crosses cells in one step, a scene that loses its numbers
 // in one) are sorted in memory by the tile's workgroup.  The list holds every
 // particle, so there is no overflow and no full sort to launch beside it.
-// What bounds it: the list's entries times the tiles (12 bytes each, from
-// L2); the host takes the radix sort instead where that is the larger (see
-// run_sort_small).  Measured at 16,384 particles: six radix launches of 41 us
+// What bounds it: the list, read by every workgroup (12 bytes an entry, from
+// L2), and the ranking of a tile's insertions; the host takes the radix sort
+// instead where that is the shorter (see run_sort_small).  Measured at 16,384 particles: six radix launches of 41 us
 // and their gaps and a grid clear of 5 us before, one of 8.6 us for both now.
 // A tile of the last order in LDS, the positions taken out of it and what is
 // put into it.

@@ -218,6 +218,7 @@ __global__ void __launch_bounds__(kScanWG) k_item_count(const uint32_t* __restri
         uint32_t moves = 0;
         if (threadIdx.x < kMoveLists) {  // one wave
             moves = plan[kPlanLists + threadIdx.x * kMoveCountStride];
+            if (!tile_net && threadIdx.x >= kSmallLists) moves = 0;  // the spilled are in their own lists' counts too
             plan[kPlanLists + threadIdx.x * kMoveCountStride] = 0u;
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) moves += __shfl_xor(moves, off, 64);

@@ -75,11 +75,14 @@ def test_batch_between_full_sorts_and_updates():
 
 
 @pytest.mark.parametrize("graph", [True, False], ids=["graph", "eager"])
-def test_small_scene_between_radix_sort_and_update(graph):
-    # 2^23 entry reads are the line: 196 tiles x 40% of 200k particles are
-    # twice that, a scene at rest reads nothing
-    sc = scenes.snow_cube(seed=9, n=200_000, res=64, lo=0.25, hi=0.5, transfer=N.PIC_FLIP, dt=1e-4,
-                          velocity=(0.4e4 / 64, 0.0, 0.0))
+@pytest.mark.parametrize("n,cells", [(16_384, 0.1), (16_384, 0.4), (100_000, 0.1), (100_000, 0.4), (200_000, 0.4),
+                                     (1_000_000, 0.02), (1_000_000, 0.1)])
+def test_small_scene_between_radix_sort_and_update(n, cells, graph):
+    # the line: a fifth of the particles, or 20,000 and a 32nd (26,250 of
+    # 200,000); then at rest
+    radix = n * cells > min(n / 5, 20000 + n / 32)
+    sc = scenes.snow_cube(seed=9, n=n, res=64, lo=0.25, hi=0.5, transfer=N.PIC_FLIP, dt=1e-4,
+                          velocity=(cells * 1e4 / 64, 0.0, 0.0))
     gpu = Solver(sc.desc, sc.particles)
     step = gpu.step_graph if graph else gpu.step
 
@@ -96,9 +99,10 @@ def test_small_scene_between_radix_sort_and_update(graph):
             assert np.array_equal(keys, ref[order]) and np.array_equal(ids, seq[order]), k
         return gpu.stats()["graph_captures"]
 
-    assert run(20) == (2 if graph else 0)
+    captures = run(20)
+    assert captures == (1 + radix if graph else 0)
     st = gpu.read_particles()
     st.velocity[:] = 0.0
     gpu.write_particles(st)
-    assert run(24) == (3 if graph else 0)
+    assert run(24) == (captures + radix if graph else 0)
     gpu.close()
