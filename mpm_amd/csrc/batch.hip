@@ -804,6 +804,7 @@ MPM_API int mpm_batch_add(void* batch, void* scene) {
     HIP_TRY(hipStreamSynchronize(s->st));
     HIP_TRY(hipStreamSynchronize(b->st));
     normalize(*b);  // before the member list changes: the new scene's pointers are its own
+    release_small_sort(*s);
     s->own_st = s->st;
     s->st = b->st;
     s->batch = b;

@@ -412,8 +412,10 @@ static void sample_moves(Solver& s) {
     const int64_t line = update_moves(s.N);
     s.update_pays = (int64_t)(uint32_t)w <= (s.update_pays ? line : line / 2);
 }
-// The buffers of the update; without them (out of memory) every step sorts
-// in full as before.
+// The buffers of the update, taken when a scene is made (its first step does
+// not wait for them); without them (out of memory) every step sorts in full
+// as before.  A member of a batch that has not stepped by itself gives them
+// back (32 bytes per particle) until it does.
 static bool ensure_small_sort(Solver& s) {
     if (s.small_sort) return true;
     if (s.incr || s.batch || s.N <= 0 || s.N >= kIncMinParticles || s.capturing) return false;
@@ -432,11 +434,20 @@ static bool ensure_small_sort(Solver& s) {
     s.moves.slot = s.moves.key + l;
     s.moves.pos = s.moves.slot + l;
     s.move_cap = small_list_cap(s.N);
-    s.history.word = pinned::take();  // without it the update is taken every time
+    if (!s.history.word) s.history.word = pinned::take();  // without it the update is taken every time
     launch_update_init(s.plan, s.moves_dev, s.moves, s.st);
     s.snap_ok = false;
     s.small_sort = true;
     return true;
+}
+void release_small_sort(Solver& s) {
+    if (!s.small_sort || s.gexec) return;  // a captured step holds the pointers
+    dfree(s, s.moves_dev);  // the one block
+    s.moves_dev = nullptr;
+    s.plan = s.snap_k = s.snap_p = nullptr;
+    s.moves = MoveList{};
+    s.small_sort = false;
+    s.snap_ok = false;
 }
 static void run_sort_small(Solver& s, const GridClear& clear) {
     ProfileHook h = hook(s);
@@ -807,6 +818,7 @@ int build(Solver& s, HostState& H, int run_init) {
         s.sort_valid = false;
         s.keys_valid = false;
     }
+    (void)ensure_small_sort(s);
     HIP_TRY(hipGetLastError());
     if (run_init) run_initialize(s);
     HIP_TRY(hipStreamSynchronize(s.st));

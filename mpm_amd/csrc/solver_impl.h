@@ -144,7 +144,7 @@ struct Solver {
     uint32_t move_cap = 0;          // capacity of one sub-list (also in the plan words)
     // a scene below kIncMinParticles: the update in one launch
     // (launch_sort_update) on the same snapshot, plan words and list (its own
-    // sub-lists; allocated at the first fused step); update_pays: shorter than
+    // sub-lists); update_pays: shorter than
     // the radix sort, by the list's length in a recent step
     bool small_sort = false;
     bool update_pays = true;
@@ -194,6 +194,7 @@ struct Scope {
 };
 void run_clear(Solver& s);
 void drop_graph(Solver& s);  // waits for its replays
+void release_small_sort(Solver& s);
 void ensure_stress(Solver& s);
 void destroy(Solver* s);
 int finish(Solver& s);

@@ -233,8 +233,12 @@ class Server:
         """The scene on the device (its own stream; safe while batch steps
         are in flight, and on a builder thread) and its measured bytes."""
         s = self.backend.create_solver(req.desc, req.particles)
+        return s, self._bytes_of(s)
+
+    @staticmethod
+    def _bytes_of(s):
         stats = getattr(s, "stats", None)
-        return s, (int(stats()["device_bytes"]) if stats is not None else None)
+        return int(stats()["device_bytes"]) if stats is not None else None
 
     def _stage(self, req: ServeRequest, rec: RequestRecord, s, nbytes):
         a = _Active(s, int(req.steps), rec, (req.desc.interp, req.desc.transfer), key_span(req.desc))
@@ -287,9 +291,12 @@ class Server:
                 self.batches[a.key] = b
                 self.batch_bytes[a.key] = 0
             b.add(a.solver)
+            nbytes = self._bytes_of(a.solver)  # a member needs no sort buffers of its own
         except N.MpmError as e:
             self._drop(a, t0, f"join failed: {e}", joined=False)
             return
+        if nbytes is not None:
+            a.bytes = nbytes
         self.active[a.rec.rid] = a
         self._measure_batch(a.key)
         self.peak_scenes = max(self.peak_scenes, len(self.active))
