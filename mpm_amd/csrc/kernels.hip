@@ -2932,63 +2932,95 @@ void launch_count_escaped(const uint32_t* sorted_keys, int64_t n, uint32_t escap
 // A workgroup takes a contiguous run of slots, scene by scene, and adds to a
 // scene's words once: they share a few cache lines, where atomics wait for
 // each other (one per wave of 64 slots: 279 us for 24 scenes of 2.6M
-// particles, 25 us now, where the 28 bytes per particle take 14).
+// particles, 25 us now, where the 28 bytes per particle take 14).  A run of more
+// than four scenes is added wave by wave, or lane by lane where a wave has
+// several: a scene's own reduction and barriers take about 1.1 us (64 scenes
+// of one particle, the whole call: 116 us scene by scene, 48 so).
+__device__ __forceinline__ int scene_of_slot(const SceneEntry* tab, int64_t i, int lo, int hi) {
+    while (lo < hi) {  // the last scene whose first slot is <= i
+        const int mid = (lo + hi + 1) >> 1;
+        if (tab[mid].pstart <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+struct HealthWords {
+    uint32_t m = 0, nb = 0, ne = 0;  // |v|^2 (as bits), non-finite, escaped
+    __device__ __forceinline__ void add(const SceneEntry& e, int64_t p, uint32_t key, uint32_t key_offset) {
+        const int64_t N = e.P.n;
+        const auto x = e.P.x, v = e.P.v;
+        const float a = v[p], b = v[N + p], c = v[2 * N + p];
+        const float x0 = x[p], x1 = x[N + p], x2 = x[2 * N + p];
+        const float sq = (a * a + b * b) + c * c;
+        const uint32_t q = __float_as_uint(sq) & 0x7FFFFFFFu;  // |v|^2 >= 0; a NaN keeps its payload above +inf
+        m = q > m ? q : m;
+        nb += (isfinite(a) && isfinite(b) && isfinite(c) && isfinite(x0) && isfinite(x1) && isfinite(x2)) ? 0u : 1u;
+        ne += key == key_offset + e.S.escape_key ? 1u : 0u;
+    }
+    __device__ __forceinline__ void merge(uint32_t om, uint32_t onb, uint32_t one) {
+        m = om > m ? om : m;
+        nb += onb;
+        ne += one;
+    }
+    __device__ __forceinline__ void reduce_wave() {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+            merge(__shfl_xor(m, off, 64), __shfl_xor(nb, off, 64), __shfl_xor(ne, off, 64));
+    }
+    __device__ __forceinline__ void put(uint32_t* out) const {
+        atomicMax(&out[0], m);
+        if (nb) atomicAdd(&out[1], nb);
+        if (ne) atomicAdd(&out[2], ne);
+    }
+};
 __global__ void __launch_bounds__(256) k_batch_health(const SceneEntry* __restrict__ tab,
                                                       const uint32_t* __restrict__ key_offsets, int ns, int64_t ntot,
                                                       int64_t per, const uint32_t* __restrict__ keys,
                                                       uint32_t* __restrict__ out) {
     __shared__ uint32_t part[4][3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int64_t i0 = (int64_t)blockIdx.x * per;
+    const int64_t i0 = (int64_t)blockIdx.x * per;
     const int64_t i1 = i0 + per < ntot ? i0 + per : ntot;
-    int sc = 0, hi = ns - 1;
-    while (sc < hi) {  // the last scene whose first slot is <= i0
-        const int mid = (sc + hi + 1) >> 1;
-        if (tab[mid].pstart <= i0) sc = mid;
-        else hi = mid - 1;
+    const int first = scene_of_slot(tab, i0, 0, ns - 1), last = scene_of_slot(tab, i1 - 1, first, ns - 1);
+    if (last - first >= 4) {  // uniform
+        for (int64_t r = i0; r < i1; r += 256) {
+            const int64_t i = r + threadIdx.x;
+            const bool act = i < i1;
+            HealthWords h;
+            int sc = last;
+            if (act) {
+                sc = scene_of_slot(tab, i, first, last);
+                h.add(tab[sc], i - tab[sc].pstart, keys[i], key_offsets[sc]);
+            }
+            const int s0 = __builtin_amdgcn_readfirstlane(sc);
+            if (__ballot(act && sc != s0) == 0ull) {
+                h.reduce_wave();
+                if (lane == 0 && act) h.put(out + 3 * s0);
+            } else if (act) {
+                h.put(out + 3 * sc);
+            }
+        }
+        return;
     }
-    for (; i0 < i1 && sc < ns; ++sc) {
-        const int64_t base = tab[sc].pstart, N = tab[sc].P.n;
-        const int64_t end = base + N < i1 ? base + N : i1;
-        if (end <= i0) continue;  // an empty scene
-        const uint32_t escape = key_offsets[sc] + tab[sc].S.escape_key;
-        const auto x = tab[sc].P.x, v = tab[sc].P.v;
-        uint32_t m = 0, nb = 0, ne = 0;
-        for (int64_t i = i0 + threadIdx.x; i < end; i += 256) {
-            const int64_t p = i - base;
-            const float a = v[p], b = v[N + p], c = v[2 * N + p];
-            const float x0 = x[p], x1 = x[N + p], x2 = x[2 * N + p];
-            const float sq = (a * a + b * b) + c * c;
-            const uint32_t q = __float_as_uint(sq) & 0x7FFFFFFFu;  // |v|^2 >= 0; a NaN keeps its payload above +inf
-            m = q > m ? q : m;
-            nb += (isfinite(a) && isfinite(b) && isfinite(c) && isfinite(x0) && isfinite(x1) && isfinite(x2)) ? 0u : 1u;
-            ne += keys[i] == escape ? 1u : 0u;
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const uint32_t o = __shfl_xor(m, off, 64);
-            m = o > m ? o : m;
-            nb += __shfl_xor(nb, off, 64);
-            ne += __shfl_xor(ne, off, 64);
-        }
+    for (int sc = first; sc <= last; ++sc) {
+        const SceneEntry& e = tab[sc];
+        const int64_t from = e.pstart > i0 ? e.pstart : i0;
+        const int64_t end = e.pstart + e.P.n < i1 ? e.pstart + e.P.n : i1;
+        if (end <= from) continue;  // an empty scene
+        HealthWords h;
+        for (int64_t i = from + threadIdx.x; i < end; i += 256) h.add(e, i - e.pstart, keys[i], key_offsets[sc]);
+        h.reduce_wave();
         if (lane == 0) {
-            part[wave][0] = m;
-            part[wave][1] = nb;
-            part[wave][2] = ne;
+            part[wave][0] = h.m;
+            part[wave][1] = h.nb;
+            part[wave][2] = h.ne;
         }
         __syncthreads();
         if (threadIdx.x == 0) {
-            for (int w = 1; w < 4; ++w) {
-                m = part[w][0] > m ? part[w][0] : m;
-                nb += part[w][1];
-                ne += part[w][2];
-            }
-            atomicMax(&out[3 * sc], m);
-            if (nb) atomicAdd(&out[3 * sc + 1], nb);
-            if (ne) atomicAdd(&out[3 * sc + 2], ne);
+            for (int w = 1; w < 4; ++w) h.merge(part[w][0], part[w][1], part[w][2]);
+            h.put(out + 3 * sc);
         }
         __syncthreads();
-        i0 = end;
     }
 }
 void launch_batch_health(const SceneEntry* tab, const uint32_t* key_offsets, int ns, int64_t ntot,
