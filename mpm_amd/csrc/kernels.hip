@@ -247,6 +247,16 @@ __global__ void __launch_bounds__(kScanWG) k_item_count(const uint32_t* __restri
     block_exclusive_scan(c, ws, tot);
     if (threadIdx.x == 0) partial[blockIdx.x] = tot;
 }
+// The last of a[lo..hi] (ascending, the first of them <= v) that is <= v.
+template <class A, class V>
+__device__ __forceinline__ int last_at_most(A a, V v, int lo, int hi) {
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (a[mid] <= v) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
 // tile_start: the scanned tile counts, or with RAW the raw counts, which
 // each workgroup sums over the tiles before it (and the last one writes the
 // item count): few tiles, one launch fewer.
@@ -283,17 +293,16 @@ __global__ void __launch_bounds__(kScanWG) k_item_emit(const uint32_t* __restric
     uint32_t tot;
     uint32_t k = first + block_exclusive_scan(c, ws, tot);
     if (RAW && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *item_count = first + tot;
-    // the scene of the tile's first key, by scalar loads; the heads go on from
-    // there (11.0M keys of 256 scenes 23 us, 36 with a search per head)
-    int sc = 0;
+    // the scenes of the tile's first and last key, by scalar loads; the heads
+    // search between them (11.0M keys of 256 scenes 23 us, 36 with a search in
+    // all scenes per head; one by one from the first, 900 scenes of one
+    // particle took 58 us longer)
+    int sc = 0, sc_last = 0;
     if (item_scene) {
-        const uint32_t key = sk[(int64_t)blockIdx.x * kScanWG * IPT];
-        int hi = nscenes - 1;
-        while (sc < hi) {
-            const int mid = (sc + hi + 1) >> 1;
-            if (key_offsets[mid] <= key) sc = mid;
-            else hi = mid - 1;
-        }
+        const int64_t i0 = (int64_t)blockIdx.x * kScanWG * IPT;
+        const int64_t i1 = i0 + kScanWG * IPT < n ? i0 + kScanWG * IPT : n;
+        sc = last_at_most(key_offsets, sk[i0], 0, nscenes - 1);
+        sc_last = last_at_most(key_offsets, sk[i1 - 1], sc, nscenes - 1);
     }
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
@@ -303,7 +312,7 @@ __global__ void __launch_bounds__(kScanWG) k_item_emit(const uint32_t* __restric
         items[k] = (uint32_t)i;
         uint32_t koff = 0;
         if (item_scene) {
-            while (sc + 1 < nscenes && key_offsets[sc + 1] <= key) ++sc;
+            sc = last_at_most(key_offsets, key, sc, sc_last);
             item_scene[k] = (uint32_t)sc;
             koff = key_offsets[sc];
         }
@@ -2357,15 +2366,13 @@ __global__ void __launch_bounds__(256) k_clear_batch(const SceneEntry* __restric
                         (kBatchClearGroups * kClearGroup);
     const int64_t gb = gb0 + lane;
     const int64_t total = block_start[nscenes];
-    int sc = 0, hi = nscenes - 1;  // the first block's scene, by scalar loads
-    while (sc < hi) {
-        const int mid = (sc + hi + 1) >> 1;
-        if (block_start[mid] <= gb0) sc = mid;
-        else hi = mid - 1;
-    }
+    // the scenes of the first and the last block, by scalar loads
+    int sc = last_at_most(block_start, gb0, 0, nscenes - 1);
+    const int64_t gb1 = gb0 + kBatchClearGroups * kClearGroup < total ? gb0 + kBatchClearGroups * kClearGroup : total;
+    const int sc_last = last_at_most(block_start, gb1 - 1, sc, nscenes - 1);
     bool t = false;
     if (gb < total) {
-        while (block_start[sc + 1] <= gb) ++sc;
+        sc = last_at_most(block_start, gb, sc, sc_last);
         const bool take = mode != 1 || tab[sc].prescat == 0u;
         t = take && clear_touched_of(tab[sc], mode)[gb - block_start[sc]] != 0u;
     }

@@ -74,3 +74,29 @@ def test_health_of_mixed_waves(sizes):
         # three roundings of the square, one of the root
         assert got["max_speed"] == speed or abs(got["max_speed"] - speed) <= 2.0**-21 * speed
     close(b, solvers)
+
+
+def test_step_of_scenes_of_one_particle():
+    # 900 scenes in one workgroup's run of keys, against 60 particles each:
+    # fewer particles are not the longer step, and the scenes are the right ones
+    one, more = make([1] * 900), make([60] * 900)
+    t = []
+    for b, _ in (one, more):
+        def steps():
+            b.step(20)
+            b.synchronize()
+        steps()
+        t.append(median_us(steps) / 20)
+    print(f"[step] 900 scenes of 1 particle {t[0]:.0f} us, of 60 particles {t[1]:.0f} us", flush=True)
+    assert t[0] < t[1]
+    for k in (0, 1, 63, 64, 450, 899):
+        alone = Solver(scenes.snow_cube(seed=k, n=1, res=8, transfer=N.APIC).desc,
+                       scenes.snow_cube(seed=k, n=1, res=8, transfer=N.APIC).particles)
+        alone.step(20 * 16)
+        x, y = one[1][k].read_particles(), alone.read_particles()
+        # one particle falls freely: 320 steps of a few 2^-24 each
+        assert np.abs(x.position.astype(np.float64) - y.position).max() <= 320 * 4 * 2.0**-24
+        assert np.abs(x.velocity.astype(np.float64) - y.velocity).max() <= 320 * 4 * 2.0**-24
+        alone.close()
+    for x in (one, more):
+        close(*x)
