@@ -368,20 +368,25 @@ void ensure_stress(Solver& s) {
     s.stress_valid = true;
 }
 
-// Once the device has written a new word (every 8 sorts; no wait), the share
-// of updates since the one before sets mostly_updates: while
-// it is 3/4 or more (or not known yet), the full sort is one launch, which
-// mostly returns at once, else it is launched pass by pass.  Where it does run
-// the one launch takes the longer (1.1M keys: 250 us against 75; 8.4M: 800
-// against 310); where it does not, 5 us against 54 and more.  Only the speed
+// The share of updates among the last 16 sorts or more (as the device wrote
+// it; no wait) sets mostly_updates: while it holds (or nothing is known yet),
+// the full sort is one launch, which mostly returns at once, else it is
+// launched pass by pass.  Where it does run the one launch takes the longer
+// (1.1M keys: 250 us against 75; 8.4M: 800 against 310); where it does not, 5
+// us against 54 and more.  So the one launch pays from a share of 0.78 (1.1M)
+// to 0.91 (8.4M): it is left below 7/8 and taken again from 15/16, apart, as a
+// captured step is captured again at each change (a reorder every third step
+// would be one change after the other at a single line).  Only the speed
 // depends on it.
 void read_history(SortHistory& h) {
     if (!h.word) return;
     const uint64_t w = __atomic_load_n(h.word, __ATOMIC_RELAXED);
     const uint32_t sorts = (uint32_t)(w >> 32), updates = (uint32_t)w;
-    if (sorts == h.sorts) return;
-    if (h.sorts != 0u)
-        h.mostly_updates = 4.0 * (double)(updates - h.updates) >= 3.0 * (double)(sorts - h.sorts);
+    if (h.sorts != 0u) {
+        const uint64_t all = sorts - h.sorts, up = updates - h.updates;
+        if (all < 2 * kHistorySorts) return;
+        h.mostly_updates = 16 * up >= (h.mostly_updates ? 14 : 15) * all;
+    }
     h.sorts = sorts;
     h.updates = updates;
 }

@@ -106,3 +106,17 @@ def test_small_scene_between_radix_sort_and_update(n, cells, graph):
     gpu.write_particles(st)
     assert run(24) == (captures + radix if graph else 0)
     gpu.close()
+
+
+@pytest.mark.parametrize("interval", [3, 5, 10])
+def test_captures_settle(interval):
+    # a reorder, and with it a full sort, every few replays: at 2/3 or 4/5
+    # updates the full sort is launched pass by pass, captured so once; at 9/10
+    # it stays the light one
+    sc = scenes.apic_slab(seed=7, nx=128, ny=64, nz=128, res=128, dt=5e-5, sigma_v=2.0)
+    gpu = Solver(sc.desc, sc.particles)
+    gpu.set_reorder_interval(interval)
+    st = replay(gpu, 120)
+    assert st["graph_captures"] == (1 if interval == 10 else 2), st
+    assert st["incremental_sorts"] >= 120 - 120 // interval - 2
+    gpu.close()
