@@ -906,8 +906,9 @@ __device__ __forceinline__ void keep_finite(bool on, float (&mx)[W], float (&rx)
 // One particle (lane src of the wave) added into the tile node by node, one
 // lane per node.  The products above multiply zeros into the components that
 // a term does not belong to, so a particle with a non-finite stress or affine
-// velocity would spread it to the others (0 * inf): it comes here instead,
-// where each component sees its own terms only.
+// velocity, or one so large that its products overflow, would spread it to the
+// others (0 * inf): it comes here instead, where each component sees its own
+// terms only.
 template <int INTERP, int APIC, int T>
 __device__ __forceinline__ void scatter_one(const SceneDev& S, f4* tile, f4* tile2, bool apart, int ox, int oy, int oz,
                                             int lane, int src, const float (&xp)[3], float mp, const float (&vp)[3],
@@ -1078,10 +1079,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P2GWave
                 const int cnt = (int)(g.e - base < 64u ? g.e - base : 64u);
                 const uint64_t tails = (heads >> 1) | (1ull << (cnt - 1));
                 const int cell = (lz * T + ly) * T + lx;
-                // finite? (a sum of some of the terms is not exactly if one is not)
-                float fin = (vs[0][1] + vs[0][2]) + (vs[1][1] + vs[1][2]) + vs[2][2];
-                if (APIC) fin += (Cm[0][1] + Cm[0][2]) + (Cm[1][1] + Cm[1][2]) + (Cm[2][1] + Cm[2][2]);
-                const uint64_t odd = __ballot(active && !__builtin_isfinite(fin));
+                // terms that are not finite, or whose products may not be (1e30
+                // leaves eight decades for h, 1 / h and the weights)
+                float big = ((fabsf(vs[0][1]) + fabsf(vs[0][2])) + (fabsf(vs[1][1]) + fabsf(vs[1][2]))) + fabsf(vs[2][2]);
+                if (APIC)
+                    big = fmaf(fmaxf(m, 1.0f),
+                               ((fabsf(Cm[0][1]) + fabsf(Cm[0][2])) + (fabsf(Cm[1][1]) + fabsf(Cm[1][2]))) +
+                                   (fabsf(Cm[2][1]) + fabsf(Cm[2][2])),
+                               big);
+                const uint64_t odd = __ballot(active && !(big < 1e30f));
                 const bool on = !((odd >> lane) & 1ull);
                 const float xp[3] = {x0, x1, x2}, vk[3] = {v0, v1, v2};
                 for (uint64_t left = odd; left; left &= left - 1)
