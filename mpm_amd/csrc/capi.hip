@@ -621,6 +621,13 @@ static GridClear take_clear(Solver& s) {
     return c;
 }
 
+// Storage blocks up to which a small scene's grid is cleared by the launch
+// that sorts: its workgroups are few at a time (the sort's LDS), so the flags
+// of a large grid take longer there than in a launch of their own.  16,384
+// particles, a whole step, in it / apart: 256^3 (2^18 blocks) 39 / 43 us, 384^3
+// 38 / 43, 512^3 (2^21) 57 / 51, 768^3 84 / 47, 1024^3 194 / 58.
+constexpr int64_t kClearWithSort = int64_t(1) << 20;
+
 void run_fused_step(Solver& s) {
     ProfileHook h = hook(s);
     const bool fuse = use_fused_transfer(s) && ensure_grid2(s) == MPM_OK;
@@ -628,7 +635,7 @@ void run_fused_step(Solver& s) {
     const bool small = ensure_small_sort(s);
     // a small scene's grid is cleared by the launch that sorts (one grid: the
     // first fused step after others may have both to clear)
-    const bool with_sort = small && !s.sort_valid;
+    const bool with_sort = small && !s.sort_valid && s.nsb <= kClearWithSort;
     GridClear clear;
     if (!scattered) {
         if (s.grid_dirty) {

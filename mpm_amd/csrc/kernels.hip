@@ -2416,9 +2416,12 @@ static unsigned grid_pass_wgs(int64_t nsb) {
 
 void launch_clear(const SceneDev& S, int64_t nsb, int nfields, unsigned long long* active, hipStream_t st) {
     if (nsb <= 0) return;
-    // enough waves to fill the device, then two groups each
+    // enough waves to fill the device, then two groups each; from two full
+    // rounds of waves with a flag per lane on (2^20 blocks) that, as most of
+    // such a grid is empty and reading its flags the work (1.2M particles in
+    // 1024^3, a whole step: 320 us with two groups, 261 with eight)
     const int64_t g = nsb / ((int64_t)kClearGroup * 32 * device_cus());
-    const int groups = g < 1 ? 1 : (g > 2 ? 2 : (int)g);
+    const int groups = g < 1 ? 1 : (g < 16 ? (g > 2 ? 2 : (int)g) : 8);
     const int64_t per = (int64_t)4 * groups * kClearGroup;  // blocks of a workgroup
     hipLaunchKernelGGL(k_clear, dim3((unsigned)((nsb + per - 1) / per)), dim3(256), 0, st, S, nsb, groups, nfields,
                        active);
