@@ -368,8 +368,8 @@ void ensure_stress(Solver& s) {
     s.stress_valid = true;
 }
 
-// The share of updates among the last 16 sorts or more (as the device wrote
-// it; no wait) sets mostly_updates: while it holds (or nothing is known yet),
+// The share of updates among the last 16 sorts or more, or the first 8 (as the
+// device wrote it; no wait), sets mostly_updates: while it holds (or nothing is known yet),
 // the full sort is one launch, which mostly returns at once, else it is
 // launched pass by pass.  Where it does run the one launch takes the longer
 // (1.1M keys: 250 us against 75; 8.4M: 800 against 310); where it does not, 5
@@ -382,11 +382,9 @@ void read_history(SortHistory& h) {
     if (!h.word) return;
     const uint64_t w = __atomic_load_n(h.word, __ATOMIC_RELAXED);
     const uint32_t sorts = (uint32_t)(w >> 32), updates = (uint32_t)w;
-    if (h.sorts != 0u) {
-        const uint64_t all = sorts - h.sorts, up = updates - h.updates;
-        if (all < 2 * kHistorySorts) return;
-        h.mostly_updates = 16 * up >= (h.mostly_updates ? 14 : 15) * all;
-    }
+    const uint64_t all = sorts - h.sorts, up = updates - h.updates;
+    if (all < (h.sorts ? 2 : 1) * kHistorySorts) return;
+    h.mostly_updates = 16 * up >= (h.mostly_updates ? 14 : 15) * all;
     h.sorts = sorts;
     h.updates = updates;
 }
