@@ -423,7 +423,7 @@ MPM_API int mpm_batch_set_reorder_interval(void* batch, int steps);
  * changed cell taken out and put back) instead of sorting in full, when
  * the list of moves fits (up to max(16384, particles / 8)); bit-identical
  * to the full sort.  On by default; 0 sorts in full every step.  The
- * single-scene counterpart is automatic (scenes of 2^20 particles and up).
+ * single-scene counterpart is automatic.
  * No reference counterpart: the reference sorts nothing, its P2G adds each
  * particle's stencil with global atomics (src/mpm_solver3d.cu:254-285). */
 MPM_API int mpm_batch_set_incremental_sort(void* batch, int enable);

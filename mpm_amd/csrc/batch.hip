@@ -621,7 +621,10 @@ int run_steps(Batch& b, int n, bool graph) {
         if (b.incr) read_history(b.history);
         if (graph && !first_scatter &&
             (!b.gexec || !(b.graph_tune == b.tune) || b.graph_light != b.history.mostly_updates)) {
-            if ((rc = capture_step(b, fused))) return rc;
+            if ((rc = capture_step(b, fused))) {
+                if (i > 0) after_steps(b, i, fused);  // the steps before it have moved the particles
+                return rc;
+            }
         }
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if (b.timing) {

@@ -402,9 +402,9 @@ void read_history(SortHistory& h) {
 //   70,000: 15% 77 / 99, 20% 86 / 99, 25% 109 / 100 (100,000: 20% 102 / 105)
 //   200,000: 10% 110 / 130, 20% 153 / 130; 400,000: 5% 150 / 173, 10% 178 / 174
 //   1,000,000: 1% 199 / 247, 5% 253 / 252, 10% 314 / 253
-// Up to about 100,000 the ranking in the tiles takes over at a fifth of the
-// particles (1,000 to 16,384 the same; 500: a half), above it the reads, about 1.6 us per
-// 1,000 moves, at what the radix sort costs more.
+// Up to about 100,000 particles the ranking in the tiles takes over at a fifth
+// of them (1,000 to 16,384 the same; 500: a half), above it the reads, about
+// 1.6 us per 1,000 moves, at what the radix sort costs more.
 // clear: a grid to clear in the same launch (cleared by its own where the
 // radix sort runs).
 static int64_t update_moves(int64_t n) { return std::max<int64_t>(250, std::min(n / 5, 20000 + n / 32)); }
@@ -1141,13 +1141,13 @@ MPM_API int mpm_step_graph(void* handle, int n) {
         if (rc) return rc;
     }
     auto t0 = std::chrono::steady_clock::now();
-    for (int i = 0; i < n; ++i) {
+    int done = 0, rc = MPM_OK;
+    for (; done < n; ++done) {
         if (reorder_due(*s)) {
             // between replays: the eager sort of the keys the last replay's
             // G2P wrote, then the permutation (the next replay sorts again)
             s->sort_valid = false;
-            int rc = reorder_store(*s);
-            if (rc) return rc;
+            if ((rc = reorder_store(*s))) break;
             if (small) seed_snapshot(*s);
             // the plan words say that the next replay sorts in full: a step
             // captured now must not hold that too, or every replay would
@@ -1157,21 +1157,27 @@ MPM_API int mpm_step_graph(void* handle, int n) {
         else if (small) sample_moves(*s);
         if (s->graph_light != s->history.mostly_updates || s->graph_update != s->update_pays) {
             drop_graph(*s);
-            const int rc = capture();
-            if (rc) return rc;
+            if ((rc = capture())) break;
         }
-        HIP_TRY(hipGraphLaunch(s->gexec, s->st));
+        const hipError_t e = hipGraphLaunch(s->gexec, s->st);
+        if (e != hipSuccess) {
+            rc = fail(MPM_ERR_HIP, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
+            break;
+        }
         s->steps += 1;
     }
-    s->version += (uint64_t)n;
-    s->grid_dirty = true;
-    s->count_on_clear = true;
-    s->vstar_dirty = false;
-    s->force_dirty = !fold;
-    s->phase = fold ? PH_FOLDED : PH_RAW;
-    s->sort_valid = false;
-    s->snap_ok = s->incr || small;
-    s->I = s->graph_I;  // a reorder between replays pointed the host copy at the identity
+    if (done > 0) {  // after an error too: the replays before it have moved the particles
+        s->version += (uint64_t)done;
+        s->grid_dirty = true;
+        s->count_on_clear = true;
+        s->vstar_dirty = false;
+        s->force_dirty = !fold;
+        s->phase = fold ? PH_FOLDED : PH_RAW;
+        s->sort_valid = false;
+        s->snap_ok = (s->incr || small) && rc == MPM_OK;
+        s->I = s->graph_I;  // a reorder between replays pointed the host copy at the identity
+    }
+    if (rc) return rc;
     auto t1 = std::chrono::steady_clock::now();
     s->last_step_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
     return finish(*s);
