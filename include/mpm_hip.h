@@ -199,7 +199,9 @@ typedef struct mpm_cache_info {
 } mpm_cache_info;
 MPM_API int mpm_set_cache_limit(int64_t bytes); /* trims every device to the new limit */
 MPM_API int mpm_get_cache_info(mpm_cache_info* out);
-/* Hands every cached block back to the driver (hipFree: waits for the device). */
+/* Hands every cached block back to the driver (hipFree: waits for the device),
+ * and the pinned words that scenes and batches report their sorts in, if none
+ * is in use. */
 MPM_API int mpm_release_cache(void);
 
 /* -------------------------------------------------------------- time steps */
@@ -211,7 +213,9 @@ MPM_API int mpm_step(void* handle, int n);
 MPM_API int mpm_synchronize(void* handle);
 
 /* Capture one simulateOneStep into a hipGraph and replay it n times
- * (identical results to mpm_step). */
+ * (identical results to mpm_step).  Asynchronous, except where the step is
+ * captured again (another form of the sort became the shorter one): that
+ * waits for the replays before it. */
 MPM_API int mpm_step_graph(void* handle, int n);
 
 /* Sub-steps, one per reference public method (include/mpm_solver3d.h:40-63).

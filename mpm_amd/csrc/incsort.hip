@@ -31,8 +31,9 @@
 // every entry's place was searched in the whole snapshot, and the removals
 // and insertions were bucketed by counts, a scan in one workgroup and a second
 // pass (searches twice as long and two launches more).  Measured, the four
-// kernels before and the two now, us: 2.1M slab 38 -> 21, 8.4M slab 85 -> 45,
-// uneven batch of 11.0M 190 -> 90, served batch of 2.6M 114 -> 47.
+// kernels before and the two now, us: 2.1M slab 38 -> 20, 8.4M slab 85 -> 47
+// (64 beside the grid's clear), uneven batch of 11.0M 190 -> 86 (114 beside the
+// clear), served batch of 2.6M 114 -> 49 (beside it).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -144,8 +144,8 @@ struct Solver {
     uint32_t move_cap = 0;          // capacity of one sub-list (also in the plan words)
     // a scene below kIncMinParticles: the update in one launch
     // (launch_sort_update) on the same snapshot, plan words and list (its own
-    // sub-lists); update_pays: shorter than
-    // the radix sort, by the list's length in a recent step
+    // sub-lists); update_pays: it is shorter than the radix sort, by the
+    // list's length in a recent step
     bool small_sort = false;
     bool update_pays = true;
     SortHistory history;
