@@ -120,3 +120,22 @@ def test_captures_settle(interval):
     assert st["graph_captures"] == (1 if interval == 10 else 2), st
     assert st["incremental_sorts"] >= 120 - 120 // interval - 2
     gpu.close()
+
+
+def test_moves_that_overflow_and_back():
+    # 0.3 cells per step of 1.1M particles: the list, then the buckets, overflow
+    # and every replay sorts in full; at rest the updates come back
+    sc = scenes.snow_cube(seed=8, n=1_100_000, res=64, lo=0.25, hi=0.5, transfer=N.PIC_FLIP, dt=1e-4,
+                          velocity=(0.3e4 / 64, 0.0, 0.0))
+    gpu = Solver(sc.desc, sc.particles)
+    gpu.set_reorder_interval(0)
+    st = replay(gpu, 20)
+    assert st["incremental_sorts"] == 0 and st["graph_captures"] == 2, st
+    check_order(gpu, sc.desc, "full sorts")
+    state = gpu.read_particles()
+    state.velocity[:] = 0.0
+    gpu.write_particles(state)
+    st = replay(gpu, 48)
+    assert st["incremental_sorts"] >= 46 and st["graph_captures"] == 3, st
+    check_order(gpu, sc.desc, "updates")
+    gpu.close()

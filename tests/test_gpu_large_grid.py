@@ -14,9 +14,9 @@ from mpm_amd.solver import Solver
 pytestmark = pytest.mark.gpu
 
 
-def step_us(n, res, dt):
+def step_us(n, res, dt, transfer=N.PIC_FLIP):
     side = (n / 8) ** (1 / 3) / res  # 8 particles per cell
-    sc = scenes.snow_cube(seed=1, n=n, res=res, lo=0.5 - side / 2, hi=0.5 + side / 2, transfer=N.PIC_FLIP, dt=dt)
+    sc = scenes.snow_cube(seed=1, n=n, res=res, lo=0.5 - side / 2, hi=0.5 + side / 2, transfer=transfer, dt=dt)
     s = Solver(sc.desc, sc.particles)
     s.step(3)
     s.synchronize()
@@ -41,3 +41,12 @@ def test_clear_of_a_mostly_empty_grid():
     # to where the body lies in the cells
     n = a["active_nodes_sum"] / a["steps"], b["active_nodes_sum"] / b["steps"]
     assert a["steps"] == b["steps"] == 183 and abs(n[0] / n[1] - 1) < 0.1
+
+
+def test_fused_transfer_in_a_mostly_empty_grid():
+    # APIC: two grids, cleared in turn beside the sort
+    _, a = step_us(16384, 64, 1e-5, N.APIC)
+    _, b = step_us(16384, 768, 1e-5, N.APIC)
+    n = a["active_nodes_sum"] / a["steps"], b["active_nodes_sum"] / b["steps"]
+    assert a["steps"] == b["steps"] == 183 and abs(n[0] / n[1] - 1) < 0.1
+    assert a["escaped"] == b["escaped"] == 0
